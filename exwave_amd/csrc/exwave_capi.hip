@@ -170,13 +170,17 @@ static void free_op(exw_op op) {
 // 1D matrices of the post-processing (layout PostTab<k>): QGauss(k+2) points
 // and weights, the Gauss-Lobatto(k+2) Lagrange basis and the QGauss(k+2)
 // collocation derivative at those points, the QGauss(k+1) (solution) basis at
-// them, and the QGauss(k+3) error rule with the Gauss-Lobatto basis there.
+// them, the QGauss(k+3) error rule with the Gauss-Lobatto basis there, and for
+// the preconditioner the eigenpairs of the 1D Laplacian D^T W D against the mass
+// W of the QGauss(k+2) points (cyclic Jacobi rotations of W^-1/2 D^T W D W^-1/2)
+// and the QGauss(k+2) basis at the Gauss-Lobatto points.
 static std::vector<double> build_post_table(int k) {
   const int N = k + 1, P = k + 2, E = k + 3;
-  std::vector<double> t(2 * P + 2 * P * P + P * N + 2 * E + E * P);
+  std::vector<double> t(2 * P + 2 * P * P + P * N + 2 * E + E * P + 2 * P * P + P);
   double xg[16], wg[16], xl[16];
   double *xq = t.data(), *wq = xq + P, *PV = wq + P, *DQ = PV + P * P, *IQ = DQ + P * P,
-         *xe = IQ + P * N, *we = xe + E, *IE = we + E;
+         *xe = IQ + P * N, *we = xe + E, *IE = we + E, *SV = IE + E * P, *LAM = SV + P * P,
+         *EG = LAM + P;
   cx::gauss01(N, xg, wg);
   cx::gauss01(P, xq, wq);
   cx::gauss_lobatto01(P, xl);
@@ -187,6 +191,44 @@ static std::vector<double> build_post_table(int k) {
     cx::lagrange(N, xg, xq[q], IQ + q * N, nullptr);
   }
   for (int q = 0; q < E; ++q) cx::lagrange(P, xl, xe[q], IE + q * P, nullptr);
+  for (int i = 0; i < P; ++i) cx::lagrange(P, xq, xl[i], EG + i * P, nullptr);
+  std::vector<double> A(P * P), V(P * P, 0.0);
+  for (int i = 0; i < P; ++i) {
+    V[i * P + i] = 1.0;
+    for (int j = 0; j < P; ++j) {
+      double s = 0.0;
+      for (int q = 0; q < P; ++q) s += wq[q] * DQ[q * P + i] * DQ[q * P + j];
+      A[i * P + j] = s / std::sqrt(wq[i] * wq[j]);
+    }
+  }
+  for (int sweep = 0; sweep < 30; ++sweep)
+    for (int p = 0; p < P; ++p)
+      for (int q = p + 1; q < P; ++q) {
+        if (A[p * P + q] == 0.0) continue;
+        const double th = (A[q * P + q] - A[p * P + p]) / (2.0 * A[p * P + q]);
+        const double tn = (th >= 0 ? 1.0 : -1.0) / (std::fabs(th) + std::sqrt(th * th + 1.0));
+        const double c = 1.0 / std::sqrt(tn * tn + 1.0), sn = tn * c;
+        for (int i = 0; i < P; ++i) {  // columns p, q of A and of the eigenvectors
+          const double a = A[i * P + p], b = A[i * P + q];
+          A[i * P + p] = c * a - sn * b;
+          A[i * P + q] = sn * a + c * b;
+          const double v = V[i * P + p], w = V[i * P + q];
+          V[i * P + p] = c * v - sn * w;
+          V[i * P + q] = sn * v + c * w;
+        }
+        for (int i = 0; i < P; ++i) {  // rows
+          const double a = A[p * P + i], b = A[q * P + i];
+          A[p * P + i] = c * a - sn * b;
+          A[q * P + i] = sn * a + c * b;
+        }
+      }
+  std::vector<int> order(P);
+  for (int m = 0; m < P; ++m) order[m] = m;
+  std::sort(order.begin(), order.end(), [&](int a, int b) { return A[a * P + a] < A[b * P + b]; });
+  for (int m = 0; m < P; ++m) {
+    LAM[m] = m == 0 ? 0.0 : A[order[m] * P + order[m]];  // the constant's eigenvalue is 0
+    for (int q = 0; q < P; ++q) SV[q * P + m] = V[q * P + order[m]] / std::sqrt(wq[q]);
+  }
   return t;
 }
 
