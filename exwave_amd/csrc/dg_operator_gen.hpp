@@ -1,6 +1,5 @@
 // dg_operator_gen.hpp -- fused operator + RK epilogue for general multilinear
-// cells of >= 48 nodes (3D k >= 3, 2D k >= 6): one cell per workgroup, one
-// lane per node, every global load issued before the first barrier.
+// cells (every degree whose cell fits a workgroup of one lane per node).
 //
 // The arithmetic is that of evaluate_cell / evaluate_inner_face /
 // evaluate_boundary_face (source/wave_equation_operations.cc:424-629) on a
@@ -8,31 +7,52 @@
 //   dv/dt = -rho^-1 J^-T grad_xi p            + lifting of the face terms
 //   dp/dt = weak div of rho c^2 w det(J) J^-1 v + lifting of the face terms
 // followed by the inverse mass 1/(w det J) (collocated Gauss basis) and the
-// RK epilogue.  How the data moves:
-//   A (lane = node): the cell's nodes; a few lanes turn the cell's corners
-//     into the coefficients of its Jacobian columns, each a bilinear (3D) or
-//     linear (2D) polynomial in the other reference coordinates;
-//   G (lane = node, then lane = face point): the node's Jacobian from those
-//     coefficients (27 FMAs in 3D instead of a sum over the 8 corners) and its
-//     inverse, the test-gradient values rho c^2 w det J (J^-1 v) (LDS), the
-//     pressure gradient and dv/dt; per face point the neighbour's nodes on
-//     the face point's line are loaded (L2 hits within the tile), the unit
-//     normal and area element are formed from the cofactors of the Jacobian
-//     there while they arrive (Nanson: det J J^-T e_d = j_{d+1} x j_{d+2}, no
-//     inverse), then the neighbour's traces and its v.n with this side's
-//     normal (LDS: 2 values per face point instead of 2 dim node-aligned
-//     fields);
-//   F (lane = face point, and lane = node): the face fluxes, and the weak
-//     divergence at the node;
-//   C (lane = node): lifting, inverse mass, epilogue with streaming stores.
-// Three barriers, no atomics.
+// RK epilogue.  Lanes alternate between flat copies, the cells' lines (a line of
+// direction d owns the two face points at its ends) and the cells' nodes:
+//   A (flat): the cells and all their neighbours in 16-byte loads; the cells go
+//     to LDS, the neighbours follow through one LDS buffer direction by
+//     direction, where (lane = line) the traces at the line's two ends are
+//     summed; a few lanes form the Jacobian column coefficients and the faces'
+//     linear flux maps meanwhile;
+//   B (lane = line): the line's nodes once from LDS: the reference gradient of
+//     p along it and the own traces at both ends; the Jacobian column along
+//     the line (constant on it) and the cofactor rows at its ends (Nanson:
+//     det J J^-T e_d = j_{d+1} x j_{d+2}), the fluxes of both face points;
+//   C (lane = node): the Jacobian from the three line columns through the
+//     node, the pressure gradient, the test-gradient values rho c^2 w det J
+//     (J^-1 v);
+//   D (lane = line): the weak derivative along the line with the lifted
+//     pressure fluxes of its two ends (still in registers);
+//   E (lane = node): velocity lifting, inverse mass, dv/dt and dp/dt over the
+//     cell's fields in LDS; (flat): the epilogue, 16 bytes at a time.
+// No atomics.
+//
+// What bounds it: the address unit takes a quad of lanes per clock, so 8-byte
+// loads and stores move 32 B per clock and CU and the neighbours' six cells at
+// that width were a third of the time (3D k=4, 33x31x29 cells: 183 us with one
+// lane per node and 8-byte gathers along the lines; 118 with the gathers left
+// out, 97 for the streaming alone).  Copied flat, 16 bytes per lane, every
+// byte costs half; the line form cuts the LDS traffic of the node form (every
+// derivative and trace re-read N values per point) to a third.  Same workload:
+// 143 us; 3D k=6 32^3 with the FP32 operator 626 -> 369 us; 3D k=2 45^3 200 ->
+// 104; 2D k=5 340^2 201 -> 118.
 #pragma once
 #include <type_traits>
 
 #include "dg_common.hpp"
+#include "gauss_cx.hpp"
 
 namespace exw {
 
+// The lanes of a group: WPD waves per direction hold its lines, so that the
+// direction is uniform over a wave and compile-time inside it (strides and
+// cofactors are constants); cells of fewer than 64 face points per direction
+// share the waves.  In the node phases lane l takes nodes l + j BLOCK, j < NPL,
+// of the group's CPB cells, in the flat copies entry pairs likewise.  Group
+// sizes as measured: half the cells per group lost 20-30 % at 3D k = 2..4 (part-
+// filled line waves), twice as many 12-60 % (fewer groups per CU); 3D k=6 lost
+// 40 % with 384 instead of its three line waves, 3D k=8 the same with six waves
+// instead of eight (two groups per CU: unevenly spread over the SIMDs).
 template <int DIM, int K>
 struct GenShape {
   static constexpr int N = K + 1;
@@ -40,64 +60,30 @@ struct GenShape {
   static constexpr int NT = DIM == 2 ? N : N * N;
   static constexpr int NF = DIM + 1;
   static constexpr int NFACE = 2 * DIM;
-  static constexpr int NFP = NFACE * NT;          // face points of a cell
-  static constexpr int BLOCK = (ND + 63) / 64 * 64;
-  static constexpr int FP_ITER = (NFP + BLOCK - 1) / BLOCK;  // face points per lane
-  // cells that fill whole waves and whose LDS fits gfx950's 160 KB
-  static constexpr int LDS_DOUBLES = (NF + DIM) * ND + NFACE * NT * (DIM + 3) + 6 * N +
-                                     2 * N * N + DIM * DIM * (1 << (DIM - 1)) + 3 * NFACE;
-  static constexpr bool ENABLED = ND >= 48 && LDS_DOUBLES * 8 <= 160 * 1024;
+  static constexpr int WPD = (NT + 63) / 64;
+  static constexpr int CPB = NT >= 64 ? 1 : 64 / NT;
+  static constexpr int LINE_LANES = DIM * WPD * 64;
+  static constexpr int NODES = CPB * ND;
+  // nodes beyond the line waves get waves of their own up to 256 lanes (512 for
+  // the cells of 512 nodes and more); degree 1 takes 256 for its copies and its
+  // few-lane tasks, which outnumber its nodes (3D 113 -> 93 us, 60^3 cells)
+  static constexpr int NODE_CAP = ND >= 512 ? 512 : 256;
+  static constexpr int NODE_LANES =
+      NODES >= NODE_CAP || K == 1 ? NODE_CAP : (NODES + 63) / 64 * 64;
+  static constexpr int BLOCK = K == 6 && DIM == 3 ? LINE_LANES
+                               : LINE_LANES > NODE_LANES ? LINE_LANES : NODE_LANES;
+  static constexpr int NPL = (NODES + BLOCK - 1) / BLOCK;
+  // node fields in LDS with rows of odd length (x lines free of bank conflicts)
+  static constexpr int NX = N % 2 ? N : N + 1;
+  static constexpr int NDP = ND / N * NX;
+  // the flat copies: PPC pairs of entries per cell, NPP per lane, all three
+  // directions' neighbours in flight where their registers allow
+  static constexpr int PPC = (NF * ND + 1) / 2, NPP = (CPB * PPC + BLOCK - 1) / BLOCK;
+  static constexpr bool PREFETCH_ALL = NPP <= 2;
+  // waves per SIMD to hold the registers to, one or two below the compiler's
+  // own choice (no spills)
+  static constexpr int MIN_WAVES = DIM == 3 ? (K <= 5 ? 5 : 4) : (K <= 3 ? 6 : 4);
 };
-
-// Column e of the Jacobian of a multilinear cell as a polynomial in the other
-// reference coordinates: with D_j = V(corner j, xi_e = 1) - V(corner j,
-// xi_e = 0) over the 2^(dim-1) corners j of the other coordinates (bit 0 of j:
-// the lower other coordinate a, bit 1: the upper one b),
-//   dx/dxi_e = D_0 + xi_a (D_1 - D_0) [+ xi_b (D_2 - D_0) + xi_a xi_b (D_3 - D_2 - D_1 + D_0)]
-// jc[e][m][i]: coefficient m of component i.  Lane (e, i) of the first DIM^2.
-template <int DIM, typename Number>
-__device__ __forceinline__ void jacobian_coefficients(const double *V, int e, int i,
-                                                      Number (*jc)[1 << (DIM - 1)][DIM]) {
-  constexpr int NJ = 1 << (DIM - 1);
-  const int a = e == 0 ? 1 : 0, b = e == 2 ? 1 : 2;  // the other coordinates (3D: a < b)
-  double D[NJ];
-#pragma unroll
-  for (int j = 0; j < NJ; ++j) {
-    const int v0 = ((j & 1) << a) | (DIM == 3 ? ((j >> 1) << b) : 0);
-    D[j] = V[(v0 | (1 << e)) * DIM + i] - V[v0 * DIM + i];
-  }
-  jc[e][0][i] = Number(D[0]);
-  jc[e][1][i] = Number(D[1] - D[0]);
-  if constexpr (DIM == 3) {
-    jc[e][2][i] = Number(D[2] - D[0]);
-    jc[e][3][i] = Number((D[3] - D[2]) - (D[1] - D[0]));
-  }
-}
-
-// J[i*DIM+e] = dx_i/dxi_e at xi from the column coefficients
-template <int DIM, typename Number>
-__device__ __forceinline__ void jacobian_eval(const Number (*jc)[1 << (DIM - 1)][DIM],
-                                              const Number *xi, Number *J) {
-#pragma unroll
-  for (int e = 0; e < DIM; ++e) {
-    // one column's coefficients at a time: an empty asm that clobbers memory
-    // keeps the compiler from loading all 2 DIM^2 NJC registers of them at
-    // once and holding them (3D k=4: 166 instead of 190 VGPRs, 3 waves per
-    // SIMD instead of 2)
-    asm volatile("" ::: "memory");
-    const int a = e == 0 ? 1 : 0, b = e == 2 ? 1 : 2;
-    const Number xa = xi[a];
-    if constexpr (DIM == 3) {
-      const Number xb = xi[b], xab = xa * xb;
-#pragma unroll
-      for (int i = 0; i < DIM; ++i)
-        J[i * DIM + e] = jc[e][0][i] + xa * jc[e][1][i] + xb * jc[e][2][i] + xab * jc[e][3][i];
-    } else {
-#pragma unroll
-      for (int i = 0; i < DIM; ++i) J[i * DIM + e] = jc[e][0][i] + xa * jc[e][1][i];
-    }
-  }
-}
 
 // Jinv[e*DIM+i] = dxi_e/dx_i of J; returns det J (as multilinear_jacobian)
 template <int DIM, typename T>
@@ -105,7 +91,7 @@ __device__ __forceinline__ T jacobian_invert(const T *J, T *Jinv) {
   T det;
   if constexpr (DIM == 2) {
     det = J[0] * J[3] - J[1] * J[2];
-    const T id = T(1) / det;
+    const T id = recip(det);
     Jinv[0] = J[3] * id;
     Jinv[1] = -J[1] * id;
     Jinv[2] = -J[2] * id;
@@ -115,7 +101,7 @@ __device__ __forceinline__ T jacobian_invert(const T *J, T *Jinv) {
             k = J[8];
     const T A = e * k - f * h, B = f * g - d * k, C = d * h - e * g;
     det = a * A + b * B + c * C;
-    const T id = T(1) / det;
+    const T id = recip(det);
     Jinv[0] = A * id;
     Jinv[3] = B * id;
     Jinv[6] = C * id;
@@ -129,322 +115,470 @@ __device__ __forceinline__ T jacobian_invert(const T *J, T *Jinv) {
   return det;
 }
 
+// 1/sqrt(x): the hardware estimate refined by Newton steps, as recip
+__device__ __forceinline__ double recip_sqrt(double x) {
+  double y = __builtin_amdgcn_rsq(x);
+#pragma unroll
+  for (int it = 0; it < 2; ++it) y = __builtin_fma(0.5 * y, __builtin_fma(-x * y, y, 1.0), y);
+  return y;
+}
+__device__ __forceinline__ float recip_sqrt(float x) {
+  const float y = __builtin_amdgcn_rsqf(x);
+  return __builtin_fmaf(0.5f * y, __builtin_fmaf(-x * y, y, 1.0f), y);
+}
+
 template <int DIM, int K, typename Number>
 __global__ void __launch_bounds__((GenShape<DIM, K>::BLOCK))
+    __attribute__((amdgpu_waves_per_eu(GenShape<DIM, K>::MIN_WAVES)))
     dg_operator_gen_kernel(const DevMesh mesh, const double *__restrict__ src,
-                           const double *__restrict__ tab, const Epilogue epi) {
+                           const Epilogue epi) {
   using S = GenShape<DIM, K>;
   constexpr int N = S::N, ND = S::ND, NT = S::NT, NF = S::NF, NFACE = S::NFACE;
-  constexpr int NFP = S::NFP, BLOCK = S::BLOCK, NV = 1 << DIM;
-  using TO = TabOff<N>;
+  constexpr int BLOCK = S::BLOCK, CPB = S::CPB, NX = S::NX, NDP = S::NDP, NV = 1 << DIM;
+  constexpr int WPD = S::WPD, NPL = S::NPL, NODES = S::NODES;
+  constexpr int PPC = S::PPC, NPP = S::NPP;
+  typedef double dbl2 __attribute__((ext_vector_type(2)));
+  typedef dbl2 dbl2u __attribute__((aligned(8)));
+  constexpr const CartConst<N> &T = CartTable<N>::value;
 
-  __shared__ Number s_u[NF][ND];
-  // per face point the neighbour's traces (v.n with this side's normal, p)
-  __shared__ Number s_tr[NFACE][NT][2];
-  __shared__ Number s_g[DIM][ND];
-  // per face point: unit outward normal and area element (A), then the face
-  // flux contributions (F writes them over its own entries)
-  __shared__ Number s_fp[NFACE][NT][DIM + 1];
-  __shared__ Number s_tab[TO::SIZE];
-  // the neighbours' materials and the Jacobian coefficients (wave-uniform
-  // values, kept in LDS rather than in registers of every lane)
-  __shared__ Number s_mat[NFACE][2];
-  __shared__ int s_nbr[NFACE];
-  __shared__ Number s_jc[DIM][1 << (DIM - 1)][DIM];
+  __shared__ Number s_u[CPB][NF][NDP];
+  // first the staged neighbour fields of one direction's two faces, then
+  // (phases B to E) the arrays below
+  struct Work {
+    // by direction: the gradient of p along it (B), the test-gradient values
+    // (C), the lines' dp/dt shares (D), each over its own entries
+    Number g[CPB][DIM][NDP];
+    Number F[CPB][NFACE][DIM][NT];  // the velocity fluxes of the face points
+    Number jd[CPB][DIM][DIM][NT];   // per line the Jacobian column along it
+  };
+  __shared__ union {
+    Number nb[2][CPB][NF][NDP];
+    Work w;
+  } s_v;
+  auto &s_g = s_v.w.g;
+  auto &s_F = s_v.w.F;
+  auto &s_jd = s_v.w.jd;
+  __shared__ Number s_jc[CPB][DIM][1 << (DIM - 1)][DIM];
+  __shared__ Number s_fc[CPB][NFACE][8];       // the faces' flux maps
+  __shared__ Number s_x[N], s_w[N], s_l[2][N];
 
   const int tid = threadIdx.x;
-  const int q = tid < ND ? tid : ND - 1;  // lanes past the last node mirror it
-  const int cell = __builtin_amdgcn_readfirstlane(xcd_remap(blockIdx.x, gridDim.x));
-  double cscale = 1.0;
-  if (epi.cell_scale) cscale = epi.cell_scale[cell];
-  const bool active = cscale != 0.0;  // uniform over the group
-  if (!active) return;
-  const size_t cbase = (size_t)cell * NF * ND;
+  const int c0 = xcd_remap(blockIdx.x, gridDim.x) * CPB;
+  // (a slot past the last cell repeats it and stores nothing)
+  auto cell_of = [&](int lc) {
+    if constexpr (CPB == 1) return c0;
+    return min(c0 + lc, mesh.n_cells - 1);
+  };
+  if constexpr (CPB == 1)
+    if (epi.cell_scale && epi.cell_scale[c0] == 0.0) return;  // uniform over the group
 
-  // ---------------- A: every global load ----------------
-  int nbr[NFACE];
-#pragma unroll
-  for (int f = 0; f < NFACE; ++f) nbr[f] = mesh.neighbor[(size_t)cell * NFACE + f];
-  double uo[NF];
-#pragma unroll
-  for (int f = 0; f < NF; ++f) uo[f] = src[cbase + f * ND + q];
-  const double rho_d = mesh.rho[cell], c_d = mesh.speed[cell];
-  if (tid < DIM * DIM)
-    jacobian_coefficients<DIM, Number>(mesh.vertices + (size_t)cell * NV * DIM, tid / DIM,
-                                       tid % DIM, s_jc);
-  if (tid < NFACE) {
-    int nb = nbr[0];
-#pragma unroll
-    for (int f = 1; f < NFACE; ++f)
-      if (tid == f) nb = nbr[f];
-    s_nbr[tid] = nb;
-    s_mat[tid][0] = Number(nb >= 0 ? mesh.rho[nb] : rho_d);
-    s_mat[tid][1] = Number(nb >= 0 ? mesh.speed[nb] : c_d);
-  }
-  for (int i = tid; i < TO::SIZE; i += BLOCK) s_tab[i] = Number(tab[i]);
-  if (tid < ND) {
-#pragma unroll
-    for (int f = 0; f < NF; ++f) s_u[f][q] = Number(uo[f]);
-  }
-  __syncthreads();  // the table, the Jacobian coefficients, the cell's fields
-  const Number rho = Number(rho_d), cc = Number(c_d);
-  const Number rho_inv = Number(1) / rho, rc2 = rho * cc * cc;
-  const Number *X = s_tab + TO::X, *W = s_tab + TO::W;
+  // the lane's line: direction dir (uniform over the wave), cell slot, line t
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int dir = wave / WPD;
+  const int li = tid - dir * (WPD * 64);
+  const int lcB = CPB == 1 ? 0 : li / NT, t = li - lcB * NT, t0 = t % N, t1 = t / N;
+  const bool line_ok = dir < DIM && (CPB == 1 ? t < NT : lcB < CPB);
+  // f(direction) at compile time, for the waves that hold lines
+  auto lines = [&](auto f) __attribute__((always_inline)) {
+    if (!line_ok) return;
+    if (dir == 0) f(std::integral_constant<int, 0>{});
+    else if (dir == 1) f(std::integral_constant<int, 1>{});
+    else if constexpr (DIM == 3) f(std::integral_constant<int, 2>{});
+  };
+  // a line's first node and stride with rows of R entries (N in memory, NX in LDS)
+  auto line_base = [&](auto D_, int R) __attribute__((always_inline)) {
+    constexpr int d = decltype(D_)::value;
+    if constexpr (DIM == 2) return d == 0 ? t * R : t;
+    else return d == 0 ? t0 * R + t1 * R * N : (d == 1 ? t0 + t1 * R * N : t0 + t1 * R);
+  };
 
-  const int qi[3] = {q % N, (q / N) % N, DIM == 3 ? q / (N * N) : 0};
-  // the node's geometry, once (registers)
-  Number Ji[DIM * DIM], jxw;
-  {
-    Number xi[DIM], J[DIM * DIM], wq = Number(1);
+  // ---------------- A ----------------
+  // the few-lane tasks (a face's flux map, a Jacobian coefficient), from the
+  // group's last lanes down (where a wave without lines is, if any): their
+  // loads first, ahead of the cells' own, finished after those are issued
+  constexpr int NT1 = CPB * NFACE, NT2 = CPB * DIM * DIM, NTASK = (NT1 + NT2 + BLOCK - 1) / BLOCK;
+  double tv[NTASK][NV / 2][2];
+  int tnb[NTASK];
 #pragma unroll
-    for (int d = 0; d < DIM; ++d) {
-      xi[d] = X[qi[d]];
-      wq *= W[qi[d]];
-    }
-    jacobian_eval<DIM>(s_jc, xi, J);
-    jxw = wq * jacobian_invert<DIM>(J, Ji);
-  }
-  if (tid < ND) {
-    // test-gradient values rho c^2 w det J (J^-1 v)_e
+  for (int j = 0; j < NTASK; ++j) {
+    const int r = BLOCK - 1 - tid + j * BLOCK;
+    tnb[j] = -1;
+    if (r < NT1) {
+      const int lc = r / NFACE, cell = cell_of(lc);
+      tnb[j] = mesh.neighbor[(size_t)cell * NFACE + (r - lc * NFACE)];
+      tv[j][0][0] = mesh.rho[cell];
+      tv[j][0][1] = mesh.speed[cell];
+    } else if (r < NT1 + NT2) {
+      const int r2 = r - NT1, lc = r2 / (DIM * DIM), ei = r2 - lc * (DIM * DIM), e = ei / DIM;
+      const double *V = mesh.vertices + (size_t)cell_of(lc) * NV * DIM + ei % DIM;
+      const int a = e == 0 ? 1 : 0, b = e == 2 ? 1 : 2;  // the other coordinates, ascending
 #pragma unroll
-    for (int e = 0; e < DIM; ++e) {
-      Number s = Number(0);
-#pragma unroll
-      for (int i = 0; i < DIM; ++i) s += Ji[e * DIM + i] * Number(uo[i]);
-      s_g[e][q] = rc2 * jxw * s;
+      for (int v = 0; v < NV / 2; ++v) {
+        const int v0 = ((v & 1) << a) | (DIM == 3 ? ((v >> 1) << b) : 0);
+        tv[j][v][0] = V[v0 * DIM];
+        tv[j][v][1] = V[(v0 | (1 << e)) * DIM];
+      }
     }
   }
-  // the cell term dv/dt = -rho^-1 J^-T grad_xi p at the node (s_u is complete)
-  const Number *D = s_tab + TO::D, *L = s_tab + TO::L;
-  Number kv[DIM];
-  {
-    Number gref[DIM];
+  // the group's cells and all their neighbours, copied as flat pairs of entries
+  // (boundary and hanging faces read the cell itself: their flux maps ignore
+  // the values)
+  dbl2 own[NPP], nbv[NPP][NFACE];
+  const double *un[NPP][NFACE], *un0[NPP];
+  int dst[NPP];  // the pair's place in a [CPB][NF][NDP] LDS array; -1: none
+#pragma unroll
+  for (int j = 0; j < NPP; ++j) {
+    const int p = tid + j * BLOCK, lc = CPB == 1 ? 0 : min(p / PPC, CPB - 1);
+    int e = 2 * (p - lc * PPC);
+    const bool ok = e < NF * ND;
+    if (!ok) e = NF * ND - 2;
+    if ((NF * ND) % 2 && e == NF * ND - 1) e = NF * ND - 2;  // (the last pair overlaps)
+    dst[j] = ok ? lc * (NF * NDP) + e / N * NX + e % N : -1;
+    const int cell = cell_of(lc);
+    const double *uc = src + (size_t)cell * (NF * ND) + e;
+#pragma unroll
+    for (int f = 0; f < NFACE; ++f) {
+      const int nb = mesh.neighbor[(size_t)cell * NFACE + f];
+      un[j][f] = src + (size_t)(nb >= 0 ? nb : cell) * (NF * ND) + e;
+    }
+    un0[j] = uc;
+    __builtin_memcpy(&own[j], uc, 16);
+  }
+  auto load_faces = [&](int d) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < NPP; ++j)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) __builtin_memcpy(&nbv[j][2 * d + s], un[j][2 * d + s], 16);
+  };
+  auto put2 = [&](Number *b, int j, dbl2 v) __attribute__((always_inline)) {
+    if (dst[j] < 0) return;
+    // (rows of odd N end between the two entries; the LDS rows are then contiguous)
+    b[dst[j]] = Number(v.x);
+    b[dst[j] + 1] = Number(v.y);
+  };
+#pragma unroll
+  for (int d = 0; d < (S::PREFETCH_ALL ? DIM : 1); ++d) load_faces(d);
+  double tm[NTASK][2];
+#pragma unroll
+  for (int j = 0; j < NTASK; ++j) {
+    const int r = BLOCK - 1 - tid + j * BLOCK;
+    if (r < NT1) {
+      const int nb = tnb[j] >= 0 ? tnb[j] : cell_of(r / NFACE);
+      tm[j][0] = mesh.rho[nb];
+      tm[j][1] = mesh.speed[nb];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < NTASK; ++j) {
+    const int r = BLOCK - 1 - tid + j * BLOCK;
+    if (r >= NT1 && r < NT1 + NT2) {
+      const int r2 = r - NT1, lc = r2 / (DIM * DIM), ei = r2 - lc * (DIM * DIM);
+      double D[NV / 2];
+#pragma unroll
+      for (int v = 0; v < NV / 2; ++v) D[v] = tv[j][v][1] - tv[j][v][0];
+      Number(*c)[DIM] = s_jc[lc][ei / DIM];
+      const int i = ei % DIM;
+      c[0][i] = Number(D[0]);
+      c[1][i] = Number(D[1] - D[0]);
+      if constexpr (DIM == 3) {
+        c[2][i] = Number(D[2] - D[0]);
+        c[3][i] = Number((D[3] - D[2]) - (D[1] - D[0]));
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < NPP; ++j) put2(&s_u[0][0][0], j, own[j]);
+  if (tid < N) {
+    s_x[tid] = Number(T.x[tid]);
+    s_w[tid] = Number(T.w[tid]);
+    s_l[0][tid] = Number(T.L[tid]);
+    s_l[1][tid] = Number(T.L[N + tid]);
+  }
+#pragma unroll
+  for (int j = 0; j < NTASK; ++j) {
+    const int r = BLOCK - 1 - tid + j * BLOCK;
+    if (r < NT1) {
+      const int lc = r / NFACE, f = r - lc * NFACE;
+      double a[4], b[4];
+      flux_matrix<double>(tv[j][0][0], tv[j][0][1], tm[j][0], tm[j][1], tnb[j] >= 0 ? 0 : -tnb[j],
+                          a, b);
+      // a hanging face contributes nothing here (nc_face_kernel adds it)
+      const double on = tnb[j] == -NC_BID ? 0.0 : 1.0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        s_fc[lc][f][i] = Number(on * a[i]);
+        s_fc[lc][f][4 + i] = Number(on * b[i]);
+      }
+    }
+  }
+  // direction by direction through LDS: the neighbours' traces at the ends of
+  // its lines, all fields
+  Number um[2][NF];
+  static_for<DIM>([&](auto R_) __attribute__((always_inline)) {
+    constexpr int r = decltype(R_)::value, lsd = r == 0 ? 1 : (r == 1 ? NX : NX * N);
+    constexpr const CartConst<N> &T = CartTable<N>::value;
+#pragma unroll
+    for (int j = 0; j < NPP; ++j)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) put2(&s_v.nb[s][0][0][0], j, nbv[j][2 * r + s]);
+    if constexpr (!S::PREFETCH_ALL && r + 1 < DIM) load_faces(r + 1);
+    __syncthreads();
+    if (line_ok && dir == r) {
+      const int lbase = line_base(R_, NX);
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+          Number a = Number(0);
+#pragma unroll
+          for (int i = 0; i < N; ++i)
+            a += Number(T.L[(1 - s) * N + i]) * s_v.nb[s][lcB][f][lbase + i * lsd];
+          um[s][f] = a;
+        }
+    }
+    __syncthreads();
+  });
+
+  // ---------------- B: lines ----------------
+  Number fp[2] = {Number(0), Number(0)};  // the pressure fluxes of the line's ends
+  lines([&](auto D_) __attribute__((always_inline)) {
+    constexpr int d = decltype(D_)::value, lsd = d == 0 ? 1 : (d == 1 ? NX : NX * N);
+    constexpr const CartConst<N> &T = CartTable<N>::value;
+    const int lbase = line_base(D_, NX);
+    Number up[2][NF];
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+      Number x[N];
+#pragma unroll
+      for (int i = 0; i < N; ++i) x[i] = s_u[lcB][f][lbase + i * lsd];
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        Number a = Number(0);
+#pragma unroll
+        for (int i = 0; i < N; ++i) a += Number(T.L[s * N + i]) * x[i];
+        up[s][f] = a;
+      }
+      if (f == DIM) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+          Number a = Number(0);
+#pragma unroll
+          for (int m = 0; m < N; ++m) a += Number(T.D[i * N + m]) * x[m];
+          s_g[lcB][d][lbase + i * lsd] = a;
+        }
+      }
+    }
+    // geometry: the column along the line, and per end the area vector
+    // sg det J J^-T e_d (|.| the area element, direction the outward normal)
+    Number jd[DIM], av[2][DIM], wt;
+    const Number(*c)[DIM] = s_jc[lcB][d];
+    if constexpr (DIM == 3) {
+      constexpr int e1 = (d + 1) % 3, e2 = (d + 2) % 3;
+      const Number xa = s_x[t0], xb = s_x[t1], xab = xa * xb;  // tangential, ascending
+      wt = s_w[t0] * s_w[t1];
+#pragma unroll
+      for (int i = 0; i < DIM; ++i) jd[i] = c[0][i] + xa * c[1][i] + xb * c[2][i] + xab * c[3][i];
+      // column e at xi_d = s and at the tangential coordinate o other than e:
+      // (c_0 + x_o c_o) + s (c_d + x_o c_3); of the two coordinates other than
+      // e the lower has coefficient 1, the upper 2
+      Number j1[2][DIM], j2[2][DIM];
+      auto ends = [&](auto E_, auto O_, Number(*j)[DIM]) __attribute__((always_inline)) {
+        constexpr int e = decltype(E_)::value, o = decltype(O_)::value;
+        constexpr int mo = o < d ? 1 : 2, md = 3 - mo;
+        const Number xo = o < e ? xa : xb;
+        const Number(*ce)[DIM] = s_jc[lcB][e];
+#pragma unroll
+        for (int i = 0; i < DIM; ++i) {
+          j[0][i] = ce[0][i] + xo * ce[mo][i];
+          j[1][i] = j[0][i] + (ce[md][i] + xo * ce[3][i]);
+        }
+      };
+      using E1 = std::integral_constant<int, e1>;
+      using E2 = std::integral_constant<int, e2>;
+      ends(E1{}, E2{}, j1);
+      ends(E2{}, E1{}, j2);
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        av[s][0] = j1[s][1] * j2[s][2] - j1[s][2] * j2[s][1];
+        av[s][1] = j1[s][2] * j2[s][0] - j1[s][0] * j2[s][2];
+        av[s][2] = j1[s][0] * j2[s][1] - j1[s][1] * j2[s][0];
+      }
+    } else {
+      const Number xa = s_x[t];
+      wt = s_w[t];
+      const Number(*ce)[DIM] = s_jc[lcB][1 - d];
+      constexpr Number turn = d == 0 ? Number(1) : Number(-1);
+#pragma unroll
+      for (int i = 0; i < DIM; ++i) jd[i] = c[0][i] + xa * c[1][i];
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        // cofactor row d: (j_1y, -j_1x) of column 1 for d = 0, (-j_0y, j_0x) for d = 1
+        av[s][0] = turn * (s ? ce[0][1] + ce[1][1] : ce[0][1]);
+        av[s][1] = -turn * (s ? ce[0][0] + ce[1][0] : ce[0][0]);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < DIM; ++i) s_jd[lcB][d][i][t] = jd[i];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      Number na2 = Number(0), det = Number(0);
+#pragma unroll
+      for (int i = 0; i < DIM; ++i) {
+        na2 += av[s][i] * av[s][i];
+        det += av[s][i] * jd[i];
+      }
+      const Number inv = recip_sqrt(na2), na = na2 * inv;
+      const Number sg = (s != 0) == (det > Number(0)) ? Number(1) : Number(-1);
+      Number vp = Number(0), vm = Number(0);
+#pragma unroll
+      for (int i = 0; i < DIM; ++i) {
+        vp += up[s][i] * av[s][i];
+        vm += um[s][i] * av[s][i];
+      }
+      vp *= sg * inv;
+      vm *= sg * inv;
+      const Number *fc = s_fc[lcB][2 * d + s];
+      const Number pn = fc[0] * vp + fc[1] * up[s][DIM] + fc[2] * vm + fc[3] * um[s][DIM];
+      const Number pp = fc[4] * vp + fc[5] * up[s][DIM] + fc[6] * vm + fc[7] * um[s][DIM];
+      const Number k = pn * sg * wt;
+#pragma unroll
+      for (int i = 0; i < DIM; ++i) s_F[lcB][2 * d + s][i][t] = k * av[s][i];
+      fp[s] = pp * na * wt;
+    }
+  });
+  __syncthreads();
+
+  // ---------------- C: nodes ----------------
+  Number kv[NPL][DIM], jxw[NPL];
+#pragma unroll
+  for (int j = 0; j < NPL; ++j) {
+    const int n = tid + j * BLOCK, lc = CPB == 1 ? 0 : n / ND, q = n - lc * ND;
+    const int qi[3] = {q % N, (q / N) % N, DIM == 3 ? q / (N * N) : 0};
+    const int ql = q / N * NX + q % N;
+    if (n >= NODES) continue;
+    const int cell = cell_of(lc);
+    const Number rho = Number(mesh.rho[cell]), cc = Number(mesh.speed[cell]);
+    Number J[DIM * DIM], Ji[DIM * DIM], wq = Number(1);
 #pragma unroll
     for (int e = 0; e < DIM; ++e) {
-      const int se = pow_n<N>(e), q0 = q - qi[e] * se;
-      Number g = Number(0);
+      const int tq = DIM == 2 ? qi[1 - e]
+                              : (e == 0 ? qi[1] + N * qi[2] : (e == 1 ? qi[0] + N * qi[2]
+                                                                      : qi[0] + N * qi[1]));
+      wq *= s_w[qi[e]];
 #pragma unroll
-      for (int m = 0; m < N; ++m) g += D[qi[e] * N + m] * s_u[DIM][q0 + m * se];
-      gref[e] = g;
+      for (int i = 0; i < DIM; ++i) J[i * DIM + e] = s_jd[lc][e][i][tq];
+    }
+    jxw[j] = wq * jacobian_invert<DIM>(J, Ji);
+    const Number rho_inv = recip(rho), gw = rho * cc * cc * jxw[j];
+    Number v[DIM];
+#pragma unroll
+    for (int i = 0; i < DIM; ++i) {
+      kv[j][i] = Number(0);
+      v[i] = s_u[lc][i][ql];
+    }
+#pragma unroll
+    for (int e = 0; e < DIM; ++e) {
+      const Number g = s_g[lc][e][ql];
+      Number a = Number(0);
+#pragma unroll
+      for (int i = 0; i < DIM; ++i) {
+        kv[j][i] += Ji[e * DIM + i] * g;
+        a += Ji[e * DIM + i] * v[i];
+      }
+      s_g[lc][e][ql] = gw * a;
     }
 #pragma unroll
     for (int i = 0; i < DIM; ++i) {
-      Number gp = Number(0);
-#pragma unroll
-      for (int e = 0; e < DIM; ++e) gp += Ji[e * DIM + i] * gref[e];
-      kv[i] = -rho_inv * gp;
-    }
-  }
-  // (empty asm that takes kv: the compiler would otherwise sink its sums
-  // into the last phase and hold the node's inverse Jacobian and gradient
-  // through the face phases, 24 registers instead of 6)
-#pragma unroll
-  for (int i = 0; i < DIM; ++i) asm volatile("" : "+v"(kv[i]));
-
-  // lane = face point: the neighbour's nodes along the face point's line are
-  // loaded first (32-bit offsets: vectors below 4 GiB), the face geometry is
-  // computed while they arrive, then the neighbour's traces of all fields and
-  // its v.n with this side's normal.
-  // Face geometry: n dA = sg det J J^-T e_d, the cofactor row d of J: in 3D
-  // the cross product j_{d+1} x j_{d+2} of the Jacobian columns, in 2D the
-  // rotated column j_{1-d}; the unit normal n = sg sign(det J) c / |c| and
-  // the area element |c| (the tangential weights are applied at the
-  // lifting).  All cofactor rows are formed and row d is selected: the face
-  // direction varies across the lanes, and selecting the operands instead
-  // would cost more selects than the two extra rows cost products.
-#pragma unroll 1
-  for (int it = 0; it < S::FP_ITER; ++it) {
-    const int fp = tid + it * BLOCK;
-    if (fp < NFP) {
-      const int f = fp / NT, t = fp - f * NT, d = f >> 1, s = f & 1;
-      int base;
-      if constexpr (DIM == 2) {
-        base = d == 0 ? t * N : t;
-      } else {
-        const int t0 = t % N, t1 = t / N;
-        base = d == 0 ? t0 * N + t1 * N * N : (d == 1 ? t0 + t1 * N * N : t0 + t1 * N);
-      }
-      const int sd = d == 0 ? 1 : (d == 1 ? N : N * N);
-      const int nb = s_nbr[f];
-      // boundary and hanging faces read the cell itself (unused values)
-      const uint32_t un = uint32_t(nb >= 0 ? nb : cell) * uint32_t(NF * ND) + uint32_t(base);
-      double gn[NF][N];
-#pragma unroll
-      for (int k = 0; k < NF; ++k)
-#pragma unroll
-        for (int i = 0; i < N; ++i) gn[k][i] = src[un + uint32_t(k * ND + i * sd)];
-
-      const Number xa = X[t % N], xb = DIM == 3 ? X[t / N] : Number(0), xs = Number(s);
-      Number xi[DIM], J[DIM * DIM];
-      if constexpr (DIM == 3) {
-        xi[0] = d == 0 ? xs : xa;
-        xi[1] = d == 0 ? xa : (d == 1 ? xs : xb);
-        xi[2] = d == 2 ? xs : xb;
-      } else {
-        xi[0] = d == 0 ? xs : xa;
-        xi[1] = d == 0 ? xa : xs;
-      }
-      jacobian_eval<DIM>(s_jc, xi, J);
-      Number c[DIM], det;
-      if constexpr (DIM == 3) {
-        Number C[3][3];
-#pragma unroll
-        for (int r = 0; r < 3; ++r) {
-          const int r1 = (r + 1) % 3, r2 = (r + 2) % 3;
-#pragma unroll
-          for (int i = 0; i < 3; ++i) {
-            const int i1 = (i + 1) % 3, i2 = (i + 2) % 3;
-            C[r][i] = J[i1 * 3 + r1] * J[i2 * 3 + r2] - J[i2 * 3 + r1] * J[i1 * 3 + r2];
-          }
-        }
-        det = J[0] * C[0][0] + J[3] * C[0][1] + J[6] * C[0][2];
-#pragma unroll
-        for (int i = 0; i < 3; ++i) c[i] = d == 0 ? C[0][i] : (d == 1 ? C[1][i] : C[2][i]);
-      } else {
-        // cofactor row d of the 2x2 Jacobian: d = 0: (J11, -J01); d = 1: (-J10, J00)
-        c[0] = d == 0 ? J[3] : -J[2];
-        c[1] = d == 0 ? -J[1] : J[0];
-        det = J[0] * J[3] - J[1] * J[2];
-      }
-      Number na = Number(0);
-#pragma unroll
-      for (int i = 0; i < DIM; ++i) na += c[i] * c[i];
-      na = sqrt(na);
-      const Number sg = (s != 0) == (det > Number(0)) ? Number(1) : Number(-1);
-      const Number inv = recip(na);
-      Number nrm[DIM];
-#pragma unroll
-      for (int i = 0; i < DIM; ++i) {
-        nrm[i] = sg * c[i] * inv;
-        s_fp[f][t][i] = nrm[i];
-      }
-      // a hanging face contributes nothing here (nc_face_kernel adds it)
-      s_fp[f][t][DIM] = nb == -NC_BID ? Number(0) : na;
-
-      const Number *Lo = L + (1 - s) * N;
-      Number an[NF];
-#pragma unroll
-      for (int k = 0; k < NF; ++k) {
-        Number a = Number(0);
-#pragma unroll
-        for (int i = 0; i < N; ++i) a += Lo[i] * Number(gn[k][i]);
-        an[k] = a;
-      }
-      Number nvm = Number(0);
-#pragma unroll
-      for (int i = 0; i < DIM; ++i) nvm += nrm[i] * an[i];
-      s_tr[f][t][0] = nvm;
-      s_tr[f][t][1] = an[DIM];
+      kv[j][i] *= -rho_inv;
+      // (not to be sunk past the barriers, which would hold J^-1 over them)
+      asm volatile("" : "+v"(kv[j][i]));
     }
   }
   __syncthreads();
 
-  // ---------------- F: face fluxes (lane = face point), weak divergence ----
-#pragma unroll 1
-  for (int it = 0; it < S::FP_ITER; ++it) {
-    const int fp = tid + it * BLOCK;
-    if (fp < NFP) {
-      const int f = fp / NT, t = fp - f * NT, d = f >> 1, s = f & 1;
-      int base;
-      if constexpr (DIM == 2) {
-        base = d == 0 ? t * N : t;
-      } else {
-        const int t0 = t % N, t1 = t / N;
-        base = d == 0 ? t0 * N + t1 * N * N : (d == 1 ? t0 + t1 * N * N : t0 + t1 * N);
-      }
-      const int sd = d == 0 ? 1 : (d == 1 ? N : N * N);
-      const Number *Ls = L + s * N;
-      // the own traces: one rolled pass along the line for all the sums (an
-      // unrolled pass keeps all its LDS loads in flight); the neighbour's
-      // from the gather phase
-      Number up[NF];
+  // ---------------- D: lines ----------------
+  // the epilogue operands, in flight during the last phases
+  dbl2 bv[NPP];
 #pragma unroll
-      for (int k = 0; k < NF; ++k) up[k] = Number(0);
-#pragma unroll 1
-      for (int i = 0; i < N; ++i) {
-        const Number ls = Ls[i];
-        const int o = base + i * sd;
+  for (int j = 0; j < NPP; ++j) {
+    bv[j] = dbl2{0.0, 0.0};
+    if (epi.b) __builtin_memcpy(&bv[j], epi.b + (un0[j] - src), 16);
+  }
+  lines([&](auto D_) __attribute__((always_inline)) {
+    constexpr int d = decltype(D_)::value, lsd = d == 0 ? 1 : (d == 1 ? NX : NX * N);
+    constexpr const CartConst<N> &T = CartTable<N>::value;
+    const int lbase = line_base(D_, NX);
+    Number x[N];
 #pragma unroll
-        for (int k = 0; k < NF; ++k) up[k] += ls * s_u[k][o];
-      }
-      const Number nvm = s_tr[f][t][0], pm = s_tr[f][t][1];
-      Number nrm[DIM], nvp = Number(0);
+    for (int i = 0; i < N; ++i) x[i] = s_g[lcB][d][lbase + i * lsd];
 #pragma unroll
-      for (int i = 0; i < DIM; ++i) {
-        nrm[i] = s_fp[f][t][i];
-        nvp += up[i] * nrm[i];
-      }
-      const Number dS = s_fp[f][t][DIM];
-      const int nb = s_nbr[f];
-      Number val_pn, val_p;
-      flux<Number>(nvp, up[DIM], nvm, pm, rho, cc, s_mat[f][0], s_mat[f][1], nb >= 0 ? 0 : -nb,
-                   val_pn, val_p);
-      // over this lane's own geometry entries (read above)
+    for (int i = 0; i < N; ++i) {
+      Number a = Number(T.L[i]) * fp[0] + Number(T.L[N + i]) * fp[1];
 #pragma unroll
-      for (int i = 0; i < DIM; ++i) s_fp[f][t][i] = val_pn * nrm[i] * dS;
-      s_fp[f][t][DIM] = val_p * dS;
+      for (int m = 0; m < N; ++m) a += Number(T.D[m * N + i]) * x[m];
+      s_g[lcB][d][lbase + i * lsd] = a;
     }
-  }
-  // the epilogue operands, in flight during the weak divergence and the last
-  // barrier (issued after the face phase)
-  double bv[NF], cv[NF];
-#pragma unroll
-  for (int f = 0; f < NF; ++f) {
-    bv[f] = epi.b ? __builtin_nontemporal_load(epi.b + cbase + f * ND + q) : 0.0;
-    cv[f] = (epi.o2 && !epi.o2_from_o1) ? __builtin_nontemporal_load(epi.c + cbase + f * ND + q)
-                                        : 0.0;
-  }
-  Number kp = Number(0);
-#pragma unroll
-  for (int e = 0; e < DIM; ++e) {
-    const int se = pow_n<N>(e), q0 = q - qi[e] * se;
-    Number a = Number(0);
-#pragma unroll
-    for (int m = 0; m < N; ++m) a += D[m * N + qi[e]] * s_g[e][q0 + m * se];
-    kp += a;
-  }
-  asm volatile("" : "+v"(kp));  // (the same for the divergence's loaded terms)
+  });
   __syncthreads();
 
-  // ---------------- C: lifting, inverse mass, epilogue ----------------
-  if (tid < ND) {
-    Number fv[DIM], fpv = Number(0);
+  // ---------------- E: nodes ----------------
+#pragma unroll
+  for (int j = 0; j < NPL; ++j) {
+    const int n = tid + j * BLOCK, lc = CPB == 1 ? 0 : n / ND, q = n - lc * ND;
+    const int qi[3] = {q % N, (q / N) % N, DIM == 3 ? q / (N * N) : 0};
+    const int ql = q / N * NX + q % N;
+    if (n >= NODES) continue;
+    Number fv[DIM], kp = Number(0);
 #pragma unroll
     for (int i = 0; i < DIM; ++i) fv[i] = Number(0);
 #pragma unroll
-    for (int d = 0; d < DIM; ++d) {
-      int t;
-      Number wt = Number(1);
-      if constexpr (DIM == 2) {
-        t = qi[1 - d];
-        wt = W[qi[1 - d]];
-      } else {
-        t = d == 0 ? qi[1] + N * qi[2] : (d == 1 ? qi[0] + N * qi[2] : qi[0] + N * qi[1]);
+    for (int e = 0; e < DIM; ++e) {
+      const int tq = DIM == 2 ? qi[1 - e]
+                              : (e == 0 ? qi[1] + N * qi[2] : (e == 1 ? qi[0] + N * qi[2]
+                                                                      : qi[0] + N * qi[1]));
+      kp += s_g[lc][e][ql];
 #pragma unroll
-        for (int e = 0; e < DIM; ++e)
-          if (e != d) wt *= W[qi[e]];
+      for (int s = 0; s < 2; ++s) {
+        const Number l = s_l[s][qi[e]];
+#pragma unroll
+        for (int i = 0; i < DIM; ++i) fv[i] += l * s_F[lc][2 * e + s][i][tq];
       }
-      const Number l0 = L[qi[d]] * wt, l1 = L[N + qi[d]] * wt;
-#pragma unroll
-      for (int i = 0; i < DIM; ++i) fv[i] += l0 * s_fp[2 * d][t][i] + l1 * s_fp[2 * d + 1][t][i];
-      fpv += l0 * s_fp[2 * d][t][DIM] + l1 * s_fp[2 * d + 1][t][DIM];
     }
-    const Number ij = Number(1) / jxw;
+    const Number ij = recip(jxw[j]);
 #pragma unroll
-    for (int i = 0; i < DIM; ++i) kv[i] += fv[i] * ij;
-    kp = (kp + fpv) * ij;
+    for (int i = 0; i < DIM; ++i) s_u[lc][i][ql] = kv[j][i] + fv[i] * ij;
+    s_u[lc][DIM][ql] = kp * ij;
+  }
+  __syncthreads();
+
+  // ---------------- epilogue, pairs of entries ----------------
+#pragma unroll
+  for (int j = 0; j < NPP; ++j) {
+    const int p = tid + j * BLOCK, lc = CPB == 1 ? 0 : min(p / PPC, CPB - 1);
+    if (dst[j] < 0 || (CPB > 1 && c0 + lc >= mesh.n_cells)) continue;
+    const double cscale = epi.cell_scale ? epi.cell_scale[c0 + lc] : 1.0;
+    if (cscale == 0.0) continue;
     const double ea1 = epi.a1 * cscale, ea2 = epi.a2 * cscale, ea3 = epi.a3 * cscale;
-#pragma unroll
-    for (int f = 0; f < NF; ++f) {
-      const size_t idx = cbase + f * ND + q;
-      const double kk = double(f < DIM ? kv[f < DIM ? f : 0] : kp);
-      const double o1 = bv[f] + ea1 * kk;
-      __builtin_nontemporal_store(o1, epi.o1 + idx);
-      if (epi.o2) {
-        const double c = epi.o2_from_o1 ? o1 : cv[f];
-        __builtin_nontemporal_store(c + ea2 * kk, epi.o2 + idx);
-        if (epi.o3) __builtin_nontemporal_store(c + ea3 * kk, epi.o3 + idx);
-      }
+    const Number *kk = &s_u[0][0][0] + dst[j];
+    const size_t idx = un0[j] - src;
+    if ((NF * ND) % 2 && p - lc * PPC == PPC - 1) {
+      // the odd last entry alone: its pair's other one belongs to the pair before
+      const size_t i = idx + 1;
+      const double k = double(kk[1]), o1 = bv[j].y + ea1 * k;
+      const double cv = epi.o2 && !epi.o2_from_o1 ? epi.c[i] : o1;
+      __builtin_nontemporal_store(o1, epi.o1 + i);
+      if (epi.o2) __builtin_nontemporal_store(cv + ea2 * k, epi.o2 + i);
+      if (epi.o2 && epi.o3) __builtin_nontemporal_store(cv + ea3 * k, epi.o3 + i);
+      continue;
+    }
+    const dbl2 k = {double(kk[0]), double(kk[1])};
+    const dbl2 o1 = bv[j] + ea1 * k;
+    dbl2 cv = o1;
+    if (epi.o2 && !epi.o2_from_o1) __builtin_memcpy(&cv, epi.c + idx, 16);
+    __builtin_nontemporal_store(o1, (dbl2u *)(epi.o1 + idx));
+    if (epi.o2) {
+      __builtin_nontemporal_store(dbl2(cv + ea2 * k), (dbl2u *)(epi.o2 + idx));
+      if (epi.o3) __builtin_nontemporal_store(dbl2(cv + ea3 * k), (dbl2u *)(epi.o3 + idx));
     }
   }
 }

@@ -9,7 +9,6 @@
 #include "dg_ader_fused.hpp"
 #include "dg_lts.hpp"
 #include "dg_misc.hpp"
-#include "dg_operator.hpp"
 #include "dg_operator_cart.hpp"
 #include "dg_operator_cartg.hpp"
 #include "dg_operator_big.hpp"
@@ -93,16 +92,6 @@ inline bool cart_pipe_enabled() {
   return on;
 }
 
-// The general-geometry kernel of one cell per group (dg_operator_gen_kernel)
-// where it applies; EXW_GEN_KERNEL=0 selects dg_operator_kernel throughout.
-inline bool gen_kernel_enabled() {
-  static const bool on = [] {
-    const char *v = getenv("EXW_GEN_KERNEL");
-    return !(v && v[0] == '0');
-  }();
-  return on;
-}
-
 // The gathered-trace Cartesian kernel (dg_operator_cartg_kernel) where it
 // applies; EXW_CART_GATHER=0 selects dg_operator_cart_kernel.  Read at every
 // launch (a scan of the environment, far below a launch's cost), so that one
@@ -177,21 +166,12 @@ hipError_t launch_op(const DevMesh &m, const double *src, const double *tab,
     hipLaunchKernelGGL((dg_operator_cart_kernel<DIM, K, Number>), dim3(grid), dim3(CS::BLOCK), 0,
                        s, m, src, e);
   } else {
-    using S = Shape<DIM, K>;
+    using G = GenShape<DIM, K>;
     if (e.cell_list) return hipErrorInvalidValue;  // cell lists: Cartesian kernel only
-    if constexpr (GenShape<DIM, K>::ENABLED) {
-      if (gen_kernel_enabled()) {
-        // one cell per group (node/face/node, geometry computed once per cell)
-        if (m.n_cells == 0) return hipSuccess;
-        hipLaunchKernelGGL((dg_operator_gen_kernel<DIM, K, Number>), dim3(m.n_cells),
-                           dim3(GenShape<DIM, K>::BLOCK), 0, s, m, src, tab, e);
-        return hipGetLastError();
-      }
-    }
-    const int grid = (m.n_cells + S::CPB - 1) / S::CPB;
+    const int grid = (m.n_cells + G::CPB - 1) / G::CPB;
     if (grid == 0) return hipSuccess;
-    hipLaunchKernelGGL((dg_operator_kernel<DIM, K, Number, CART>), dim3(grid), dim3(S::BLOCK), 0,
-                       s, m, src, tab, e);
+    hipLaunchKernelGGL((dg_operator_gen_kernel<DIM, K, Number>), dim3(grid), dim3(G::BLOCK), 0, s,
+                       m, src, e);
   }
   return hipGetLastError();
 }
