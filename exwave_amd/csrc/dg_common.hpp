@@ -196,8 +196,30 @@ __device__ __forceinline__ double recip(double x) {
 }
 __device__ __forceinline__ float recip(float x) { return 1.0f / x; }
 
+// The kernels of one sweep must agree in every bit (the pipelined, gathered
+// and fused forms against the plain one), so what each of them evaluates in code
+// of its own says which products are fused: explicit FMAs, and no contraction
+// elsewhere (left to itself the compiler fuses a b + c d either way, by context).
+__device__ __forceinline__ double fma_of(double a, double b, double c) {
+  return __builtin_fma(a, b, c);
+}
+__device__ __forceinline__ float fma_of(float a, float b, float c) {
+  return __builtin_fmaf(a, b, c);
+}
+// one row of a face's flux map on (own v_n, own p, neighbour v_n, neighbour p)
+template <typename T>
+__device__ __forceinline__ T flux_row(const T *c, T vo, T po, T vn, T pn) {
+  return fma_of(c[3], pn, fma_of(c[2], vn, fma_of(c[1], po, c[0] * vo)));
+}
+// k plus the lifting of the two face values of a line
+template <typename T>
+__device__ __forceinline__ T lift_ends(T k, T l0, T f0, T l1, T f1) {
+  return fma_of(l1, f1, fma_of(l0, f0, k));
+}
+
 template <typename T>
 __device__ __forceinline__ void flux_lambda(T rho_p, T c_p, T rho_m, T c_m, int bid, T *l) {
+#pragma clang fp contract(off)
   const T tau_p = recip(c_p * rho_p);
   l[0] = l[1] = l[2] = l[3] = T(0);
   if (bid == 0) {
@@ -241,6 +263,7 @@ __device__ __forceinline__ void flux(T nvp, T pp, T nv_m, T pm, T rho_p, T c_p, 
 // p) -> (v test value, p test value): a[j], b[j] multiply input j.
 template <typename T>
 __device__ __forceinline__ void flux_matrix(T rho_p, T c_p, T rho_m, T c_m, int bid, T *a, T *b) {
+#pragma clang fp contract(off)
   T l[4];
   flux_lambda<T>(rho_p, c_p, rho_m, c_m, bid, l);
   const T irho = recip(rho_p), tau_p = recip(c_p * rho_p), z = c_p * c_p * rho_p;

@@ -23,8 +23,7 @@
 // Global traffic is coalesced exactly like a streaming kernel; LDS traffic is
 // one read + one write per value and line instead of N reads per derivative.
 #pragma once
-#include "dg_common.hpp"
-#include "gauss_cx.hpp"
+#include "dg_operator_gen.hpp"
 
 namespace exw {
 
@@ -232,13 +231,13 @@ __device__ __forceinline__ void cart_cell(const DevMesh &mesh, const double *__r
         pn += lo * s_nb[lcB][f][1][n];
       }
       const Number *c = s_fc[lcB][f];
-      const Number fv = c[0] * vo + c[1] * po + c[2] * vn + c[3] * pn;
-      const Number fp = c[4] * vo + c[5] * po + c[6] * vn + c[7] * pn;
+      const Number fv = flux_row(c, vo, po, vn, pn);
+      const Number fp = flux_row(c + 4, vo, po, vn, pn);
 #pragma unroll
       for (int i = 0; i < N; ++i) {
         const Number lw = Number(T.LW[s * N + i]);
-        kv[i] += lw * fv;
-        kp[i] += lw * fp;
+        kv[i] = fma_of(lw, fv, kv[i]);
+        kp[i] = fma_of(lw, fp, kp[i]);
       }
     }
 #pragma unroll
@@ -275,10 +274,6 @@ __global__ void __launch_bounds__((CartShape<DIM, K>::BLOCK))
   constexpr int ND = S::ND, NF = S::NF, LANES = S::LANES;
   static_assert(S::ITER == 1, "one cell per lane slot and group");
   __shared__ CartLds<DIM, K, Number> lds;
-#ifdef EXW_LDS_PAD
-  __shared__ double s_pad[EXW_LDS_PAD];
-  if (threadIdx.x == 1023) s_pad[0] = 0.0;
-#endif
   int lc, cell;
   bool active;
   double cscale, bv[NF];
@@ -301,6 +296,323 @@ __global__ void __launch_bounds__((CartShape<DIM, K>::BLOCK))
         const double cv = epi.o2_from_o1 ? o1 : epi.c[idx];
         __builtin_nontemporal_store(cv + ea2 * kk, epi.o2 + idx);
         if (epi.o3) __builtin_nontemporal_store(cv + ea3 * kk, epi.o3 + idx);
+      }
+    }
+  }
+}
+
+// dg_operator_cartp_kernel: the same sweep for large launches of small cells,
+// everything that touches memory in 16-byte pairs of entries.  The address unit
+// takes a quad of lanes per clock, so the 8-byte accesses of one lane per node
+// cost twice the time of pairs, and cells of a few nodes fill the node-aligned
+// lanes badly (2D k=5: 36 lines on a group's 128 lanes).  Here the cells, their
+// neighbours' fields, the accumulator and the outputs are flat copies, and the
+// lines have GenShape's line waves (direction uniform per wave).  It costs more
+// barriers than dg_operator_cart_kernel (all neighbour fields of the group
+// staged at once where they take up to 24 KB, FULL; else one direction's at a
+// time) and larger groups, so it pays where memory accesses dominate.
+// RK stage, us, dg_operator_cart_kernel -> this one: 2D 301x287 k=5 102 -> 80,
+// 512^2 k=3 109 -> 93, 700^2 k=2 192 -> 168, 1000^2 k=1 186 -> 111; 3D 45^3 k=2
+// 109 -> 99, 60^3 k=1 97 -> 62, FP32 40^3 k=4 250 -> 219.
+// Where it was measured faster: sweeps with two outputs and more (with one the
+// staged kernel moves too little to gain, and lost nowhere but at 2D k=5), on at
+// least one group per CU (below, both take their latency, and the staged one's
+// smaller groups spread better: 2D k=4 32^2 6.1 against 7.3 us; degree 1 always
+// gains), for 2D but k=6 (123 against 131 us, FP32), 3D k <= 2, and 3D k=4, 5 with
+// the FP32 operator (FP64 runs the pipelined kernel there; k=3: 116 against 119).
+template <int DIM, int K, typename Number>
+constexpr bool cart_pairs_pay() {
+  return DIM == 2 ? K != 6 : (K <= 2 || (std::is_same_v<Number, float> && (K == 4 || K == 5)));
+}
+
+template <int DIM, int K, typename Number>
+struct CartLines {
+  using G = GenShape<DIM, K>;
+  static constexpr int N = G::N, ND = G::ND, NF = G::NF, NFACE = G::NFACE, CPB = G::CPB;
+  static constexpr int BLOCK = G::BLOCK, NDP = G::NDP;
+  // the staged fields: PPF pairs of entries per field, one direction's two faces
+  // with two fields each per round
+  static constexpr int PPF = (ND + 1) / 2;
+  static constexpr int NPF = (CPB * 4 * PPF + BLOCK - 1) / BLOCK;
+  static constexpr int FULL_BYTES = CPB * (NF + 2 * NFACE) * NDP * int(sizeof(Number));
+  static constexpr bool FULL = FULL_BYTES <= 24 * 1024;
+  static constexpr int ROUND_FIELDS = FULL ? 2 * NFACE : 4;
+};
+
+template <int DIM, int K, typename Number>
+__global__ void __launch_bounds__((CartLines<DIM, K, Number>::BLOCK))
+    dg_operator_cartp_kernel(const DevMesh mesh, const double *__restrict__ src,
+                            const Epilogue epi) {
+  using S = GenShape<DIM, K>;
+  using C = CartLines<DIM, K, Number>;
+  constexpr int N = S::N, ND = S::ND, NT = S::NT, NF = S::NF, NFACE = S::NFACE;
+  constexpr int BLOCK = S::BLOCK, CPB = S::CPB, NX = S::NX, NDP = S::NDP, WPD = S::WPD;
+  constexpr int PPC = S::PPC, NPP = S::NPP, PPF = C::PPF, NPF = C::NPF;
+  constexpr bool FULL = C::FULL;
+  typedef double dbl2 __attribute__((ext_vector_type(2)));
+  typedef dbl2 dbl2u __attribute__((aligned(8)));
+
+  __shared__ Number s_u[CPB][NF][NDP];
+  // the neighbours' v_n (0) and p (1) of faces 2d + s, as [d][s][0/1] (FULL) or of
+  // the round's direction as [s][0/1]; then the lines' dp/dt shares: direction d's
+  // over [d][0][1] (FULL: its own lines' entries) or [d]
+  __shared__ Number s_nb[C::ROUND_FIELDS][CPB][NDP];
+  __shared__ Number s_fc[CPB][NFACE][8];
+  __shared__ Number s_vc[CPB][DIM][2];
+  auto kp_slot = [](int d) { return FULL ? 4 * d + 1 : d; };
+
+  const int tid = threadIdx.x;
+  const int c0 = xcd_remap(blockIdx.x, gridDim.x) * CPB;
+  const int n_entries = epi.cell_list ? epi.n_list : mesh.n_cells;
+  // (a slot past the last entry repeats it and stores nothing)
+  auto cell_of = [&](int lc) __attribute__((always_inline)) {
+    const int e = CPB == 1 ? c0 : min(c0 + lc, n_entries - 1);
+    return epi.cell_list ? epi.cell_list[e] : e;
+  };
+  if constexpr (CPB == 1)
+    if (epi.cell_scale && epi.cell_scale[cell_of(0)] == 0.0) return;  // uniform over the group
+
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int dir = wave / WPD;
+  const int li = tid - dir * (WPD * 64);
+  const int lcB = CPB == 1 ? 0 : li / NT, t = li - lcB * NT, t0 = t % N, t1 = t / N;
+  const bool line_ok = dir < DIM && (CPB == 1 ? t < NT : lcB < CPB);
+  auto line_base = [&](auto D_) __attribute__((always_inline)) {
+    constexpr int d = decltype(D_)::value;
+    if constexpr (DIM == 2) return d == 0 ? t * NX : t;
+    else return d == 0 ? t0 * NX + t1 * NX * N : (d == 1 ? t0 + t1 * NX * N : t0 + t1 * NX);
+  };
+
+  // ---------------- A ----------------
+  // the faces' flux maps, one lane each from the group's last lanes down: their
+  // loads first, ahead of the cells' own
+  constexpr int NT1 = CPB * NFACE, NTASK = (NT1 + BLOCK - 1) / BLOCK;
+  double tv[NTASK][5];
+  int tnb[NTASK];
+#pragma unroll
+  for (int j = 0; j < NTASK; ++j) {
+    const int r = BLOCK - 1 - tid + j * BLOCK;
+    tnb[j] = -1;
+    if (r < NT1) {
+      const int lc = r / NFACE, f = r - lc * NFACE, cell = cell_of(lc);
+      tnb[j] = mesh.neighbor[(size_t)cell * NFACE + f];
+      tv[j][0] = mesh.rho[cell];
+      tv[j][1] = mesh.speed[cell];
+      tv[j][4] = mesh.h[(size_t)cell * DIM + (f >> 1)];
+    }
+  }
+  // the cells, flat, 16 bytes per lane
+  dbl2 own[NPP];
+  size_t idx[NPP];  // the pair's place in the vectors
+  int dst[NPP];     // and in s_u; -1: none
+#pragma unroll
+  for (int j = 0; j < NPP; ++j) {
+    const int p = tid + j * BLOCK, lc = CPB == 1 ? 0 : min(p / PPC, CPB - 1);
+    int e = 2 * (p - lc * PPC);
+    const bool ok = e < NF * ND;
+    if (!ok || ((NF * ND) % 2 && e == NF * ND - 1)) e = NF * ND - 2;  // (the odd last pair overlaps)
+    dst[j] = ok ? lc * (NF * NDP) + e / N * NX + e % N : -1;
+    idx[j] = (size_t)cell_of(lc) * (NF * ND) + e;
+    __builtin_memcpy(&own[j], src + idx[j], 16);
+  }
+  // the neighbours' fields of direction d's faces, flat per field (boundary and
+  // hanging faces read the cell itself: their flux maps ignore the values)
+  dbl2 nbv[DIM][NPF];
+  auto load_faces = [&](int d) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < NPF; ++j) {
+      const int q = tid + j * BLOCK, g = min(q / PPF, 4 * CPB - 1);  // field g of the round
+      const int lc = g / 4, s = (g >> 1) & 1, c = g & 1;
+      int e = 2 * min(q - g * PPF, PPF - 1);
+      if (ND % 2 && e == ND - 1) e = ND - 2;
+      const int cell = cell_of(lc), nb = mesh.neighbor[(size_t)cell * NFACE + 2 * d + s];
+      const double *un = src + (size_t)(nb >= 0 ? nb : cell) * (NF * ND) + (c ? DIM : d) * ND + e;
+      __builtin_memcpy(&nbv[d][j], un, 16);
+    }
+  };
+  auto put_faces = [&](int d) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < NPF; ++j) {
+      const int q = tid + j * BLOCK, g = q / PPF;
+      int e = 2 * (q - g * PPF);
+      if (ND % 2 && e == ND - 1) e = ND - 2;
+      if (g < 4 * CPB) {
+        Number *o = &s_nb[(FULL ? 4 * d : 0) + (g & 3)][g >> 2][e / N * NX + e % N];
+        o[0] = Number(nbv[d][j].x);
+        o[1] = Number(nbv[d][j].y);
+      }
+    }
+  };
+#pragma unroll
+  for (int d = 0; d < DIM; ++d) load_faces(d);
+  double tm[NTASK][2];
+#pragma unroll
+  for (int j = 0; j < NTASK; ++j) {
+    const int r = BLOCK - 1 - tid + j * BLOCK;
+    if (r < NT1) {
+      const int nb = tnb[j] >= 0 ? tnb[j] : cell_of(r / NFACE);
+      tm[j][0] = mesh.rho[nb];
+      tm[j][1] = mesh.speed[nb];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < NPP; ++j)
+    if (dst[j] >= 0) {
+      Number *o = &s_u[0][0][0] + dst[j];
+      o[0] = Number(own[j].x);
+      o[1] = Number(own[j].y);
+    }
+#pragma unroll
+  for (int j = 0; j < NTASK; ++j) {
+    const int r = BLOCK - 1 - tid + j * BLOCK;
+    if (r < NT1) {
+      // columns of the linear flux map (evaluate_inner_face /
+      // evaluate_boundary_face, source/wave_equation_operations.cc:480-629)
+      const int lc = r / NFACE, f = r - lc * NFACE, d = f >> 1, nb = tnb[j];
+      const double rho = tv[j][0], cc = tv[j][1];
+      const double ih = recip(tv[j][4]);
+      const double sg = (f & 1) ? 1.0 : -1.0;
+      // a hanging face contributes nothing here (nc_face_kernel adds it)
+      const double ihf = nb == -NC_BID ? 0.0 : ih;
+      double a[4], b[4];
+      flux_matrix<double>(rho, cc, tm[j][0], tm[j][1], nb >= 0 ? 0 : -nb, a, b);
+      // inputs (v_d, p, neighbour v_d, neighbour p): v.n = sg v_d on both sides
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const double in = (i == 0 || i == 2) ? sg : 1.0;
+        s_fc[lc][f][i] = Number(a[i] * in * sg * ihf);
+        s_fc[lc][f][4 + i] = Number(b[i] * in * ihf);
+      }
+      if ((f & 1) == 0) {  // the cell term's factors of direction d
+        s_vc[lc][d][0] = Number(-ih * recip(rho));
+        s_vc[lc][d][1] = Number(rho * cc * cc * ih);
+      }
+    }
+  }
+  Number tr[2][2];  // the neighbours' traces (v_n, p) at the line's ends
+  auto traces = [&](auto D_) __attribute__((always_inline)) {
+    constexpr int d = decltype(D_)::value, sd = d == 0 ? 1 : (d == 1 ? NX : NX * N);
+    constexpr const CartConst<N> &T = CartTable<N>::value;
+    const int base = line_base(D_);
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const Number *x = s_nb[(FULL ? 4 * d : 0) + 2 * s + c][lcB] + base;
+        Number a = Number(0);
+#pragma unroll
+        for (int i = 0; i < N; ++i) a += Number(T.L[(1 - s) * N + i]) * x[i * sd];
+        tr[s][c] = a;
+      }
+  };
+  if constexpr (FULL) {
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) put_faces(d);
+    __syncthreads();
+  } else {
+    static_for<DIM>([&](auto R_) __attribute__((always_inline)) {
+      put_faces(decltype(R_)::value);
+      __syncthreads();
+      if (line_ok && dir == decltype(R_)::value) traces(R_);
+      __syncthreads();
+    });
+  }
+  // the accumulator, in flight during the line phase
+  dbl2 bv[NPP];
+#pragma unroll
+  for (int j = 0; j < NPP; ++j) {
+    bv[j] = dbl2{0.0, 0.0};
+    if (epi.b) bv[j] = __builtin_nontemporal_load((const dbl2u *)(epi.b + idx[j]));
+  }
+
+  // ---------------- B: one lane per line ----------------
+  static_for<DIM>([&](auto D_) __attribute__((always_inline)) {
+    constexpr int d = decltype(D_)::value, sd = d == 0 ? 1 : (d == 1 ? NX : NX * N);
+    constexpr const CartConst<N> &T = CartTable<N>::value;
+    if (!line_ok || dir != d) return;
+    if constexpr (FULL) traces(D_);
+    const int base = line_base(D_);
+    const Number cvv = s_vc[lcB][d][0], cvp = s_vc[lcB][d][1];
+    Number vl[N], pl[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      vl[i] = s_u[lcB][d][base + i * sd];
+      pl[i] = s_u[lcB][DIM][base + i * sd];
+    }
+    Number fv[2], fp[2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      Number vo = Number(0), po = Number(0);
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        vo += Number(T.L[s * N + i]) * vl[i];
+        po += Number(T.L[s * N + i]) * pl[i];
+      }
+      const Number *c = s_fc[lcB][2 * d + s];
+      fv[s] = flux_row(c, vo, po, tr[s][0], tr[s][1]);
+      fp[s] = flux_row(c + 4, vo, po, tr[s][0], tr[s][1]);
+    }
+    Number(*ks)[NDP] = s_nb[kp_slot(d)];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      Number dv = Number(0);
+#pragma unroll
+      for (int m = 0; m < N; ++m) dv += Number(T.DT[i * N + m]) * vl[m];
+      const Number k = lift_ends(cvp * dv, Number(T.LW[i]), fp[0], Number(T.LW[N + i]), fp[1]);
+      ks[lcB][base + i * sd] = k;
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      Number gp = Number(0);
+#pragma unroll
+      for (int m = 0; m < N; ++m) gp += Number(T.D[i * N + m]) * pl[m];
+      const Number k = lift_ends(cvv * gp, Number(T.LW[i]), fv[0], Number(T.LW[N + i]), fv[1]);
+      s_u[lcB][d][base + i * sd] = k;  // (over v_d, which only this lane reads)
+    }
+  });
+  __syncthreads();
+
+  // ---------------- C: fused epilogue, pairs of entries ----------------
+  // M^-1 A(src) at entry e (LDS place l) of a cell
+  auto value = [&](int lc, int e, int l) __attribute__((always_inline)) {
+    if (e < DIM * ND) return double((&s_u[0][0][0])[l]);
+    const int n = l - lc * (NF * NDP) - DIM * NDP;
+    Number kp = s_nb[kp_slot(0)][lc][n];
+#pragma unroll
+    for (int d = 1; d < DIM; ++d) kp += s_nb[kp_slot(d)][lc][n];
+    return double(kp);
+  };
+#pragma unroll
+  for (int j = 0; j < NPP; ++j) {
+    const int p = tid + j * BLOCK, lc = CPB == 1 ? 0 : min(p / PPC, CPB - 1);
+    if (dst[j] < 0 || (CPB > 1 && c0 + lc >= n_entries)) continue;
+    const double cscale = epi.cell_scale ? epi.cell_scale[cell_of(lc)] : 1.0;
+    if (cscale == 0.0) continue;
+    const double ea1 = epi.a1 * cscale, ea2 = epi.a2 * cscale, ea3 = epi.a3 * cscale;
+    const bool odd = (NF * ND) % 2 && p - lc * PPC == PPC - 1;
+    const int e = odd ? NF * ND - 2 : 2 * (p - lc * PPC);
+    const double k1 = value(lc, e + 1, dst[j] + 1);
+    if (odd) {
+      // the odd last entry alone: its pair's other one belongs to the pair before
+      const size_t i = idx[j] + 1;
+      const double o1 = bv[j].y + ea1 * k1;
+      const double cv = epi.o2 && !epi.o2_from_o1 ? epi.c[i] : o1;
+      __builtin_nontemporal_store(o1, epi.o1 + i);
+      if (epi.o2) __builtin_nontemporal_store(cv + ea2 * k1, epi.o2 + i);
+      if (epi.o2 && epi.o3) __builtin_nontemporal_store(cv + ea3 * k1, epi.o3 + i);
+      continue;
+    }
+    const double k0 = value(lc, e, dst[j]);
+    const dbl2 o1 = {bv[j].x + ea1 * k0, bv[j].y + ea1 * k1};
+    dbl2 cv = o1;
+    if (epi.o2 && !epi.o2_from_o1) __builtin_memcpy(&cv, epi.c + idx[j], 16);
+    __builtin_nontemporal_store(o1, (dbl2u *)(epi.o1 + idx[j]));
+    if (epi.o2) {
+      const dbl2 o2 = {cv.x + ea2 * k0, cv.y + ea2 * k1};
+      __builtin_nontemporal_store(o2, (dbl2u *)(epi.o2 + idx[j]));
+      if (epi.o3) {
+        const dbl2 o3 = {cv.x + ea3 * k0, cv.y + ea3 * k1};
+        __builtin_nontemporal_store(o3, (dbl2u *)(epi.o3 + idx[j]));
       }
     }
   }

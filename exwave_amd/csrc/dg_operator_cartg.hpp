@@ -247,8 +247,8 @@ __global__ void __launch_bounds__((CartGShape<DIM, K>::BLOCK))
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
         const Number *c = s_fc[2 * d + s];
-        fv[s] = c[0] * vo[s] + c[1] * po[s] + c[2] * tv[s] + c[3] * tp[s];
-        fp[s] = c[4] * vo[s] + c[5] * po[s] + c[6] * tv[s] + c[7] * tp[s];
+        fv[s] = flux_row(c, vo[s], po[s], tv[s], tp[s]);
+        fp[s] = flux_row(c + 4, vo[s], po[s], tv[s], tp[s]);
       }
     }
     asm volatile("" ::: "memory");  // reload, do not keep the first loads
@@ -261,9 +261,7 @@ __global__ void __launch_bounds__((CartGShape<DIM, K>::BLOCK))
         Number dv = Number(0);
 #pragma unroll
         for (int m = 0; m < N; ++m) dv += Number(T.DT[i * N + m]) * vl[m];
-        Number k = cvp * dv;
-        k += Number(T.LW[i]) * fp[0];
-        k += Number(T.LW[N + i]) * fp[1];
+        const Number k = lift_ends(cvp * dv, Number(T.LW[i]), fp[0], Number(T.LW[N + i]), fp[1]);
         s_kp[d][base + i * sd] = k;
       }
     }
@@ -277,9 +275,7 @@ __global__ void __launch_bounds__((CartGShape<DIM, K>::BLOCK))
         Number gp = Number(0);
 #pragma unroll
         for (int m = 0; m < N; ++m) gp += Number(T.D[i * N + m]) * pl[m];
-        Number k = cvv * gp;
-        k += Number(T.LW[i]) * fv[0];
-        k += Number(T.LW[N + i]) * fv[1];
+        const Number k = lift_ends(cvv * gp, Number(T.LW[i]), fv[0], Number(T.LW[N + i]), fv[1]);
         s_u[d][base + i * sd] = k;
       }
     }
