@@ -15,7 +15,7 @@
 // so n steps through this kernel give the bits of n exw_ader_step calls.
 //
 // What it saves: the CK kernel's read of u_n+1 and one launch per step, and
-// -- the point -- the CK's LDS-bound arithmetic overlaps the sweep's memory
+// -- the point -- the CK's arithmetic overlaps the sweep's memory
 // traffic of other groups on the same CU instead of running in a kernel of
 // its own.  Cartesian cells whose sweep and CK groups coincide (3D k = 3..5);
 // FP64 runs ader_sweepg_ck_kernel (below) instead, whose sweep half
@@ -30,37 +30,60 @@ namespace exw {
 template <int DIM, int K>
 struct AderFusedShape {
   using CS = CartShape<DIM, K>;
-  using G = CkGroup<DIM, K>;
   static constexpr int CPB = CS::CPB, BLOCK = CS::BLOCK;
-  static constexpr int LOW = CkShape<K>::low_off(DIM, CkShape<K>::N_LEVELS) > 0
-                                 ? CkShape<K>::low_off(DIM, CkShape<K>::N_LEVELS)
-                                 : 1;
-  // the two kernels' groups hold the same cells on the same lanes
+  static constexpr int LANES = CS::LANES;  // per cell, whole waves
   static constexpr bool ENABLED =
-      DIM == 3 && K >= 3 && K <= 5 && CS::ITER == 1 && CS::CPB == G::CPB && CS::BLOCK == G::BLOCK;
+      DIM == 3 && K >= 3 && K <= 5 && CS::ITER == 1 && CS::NLINE <= LANES && CPB * LANES == BLOCK;
 };
+
+// The CK half of the fused kernels: LDS and the work of the group's cells once
+// node lane lt < ND of cell slot lc holds the new state un (swept: the slot's
+// cell exists).  LANES lanes per cell, line lanes first.
+template <int DIM, int K, typename Number, int CPB>
+struct AderFusedCk {
+  static constexpr int LD = CkGrid<DIM, K + 1>::SIZE;
+  Number a[CPB][DIM + 1][LD];
+  Number b[CPB][DIM][LD];
+};
+template <int DIM, int K, typename Number, int CPB>
+__device__ __forceinline__ void fused_ck(AderFusedCk<DIM, K, Number, CPB> &L, const DevMesh &mesh,
+                                         int cell, int lc, int lt, bool swept,
+                                         const double (&un)[DIM + 1], double dt,
+                                         double *__restrict__ w_out) {
+  constexpr int N = K + 1, NT = DIM == 2 ? N : N * N, ND = Shape<DIM, K>::ND, NF = DIM + 1;
+  const int q = CkGrid<DIM, N>::node(lt);
+  if (swept && lt < ND) {
+#pragma unroll
+    for (int f = 0; f < NF; ++f) L.a[lc][f][q] = Number(un[f]);
+  }
+  const bool ok = lt < DIM * NT;
+  const int d = ok ? small_div<NT>(lt) : 0, t = ok ? lt - d * NT : 0;
+  const Number rho = Number(mesh.rho[cell]), cc = Number(mesh.speed[cell]);
+  const Number ih = recip(Number(mesh.h[(size_t)cell * DIM + d]));
+  __syncthreads();
+  ck_lines<DIM, K, Number>(L.a[lc][0], L.b[lc][0], ok, d, t, recip(rho) * ih, (rho * cc * cc) * ih, dt,
+                           0.0, 0.0, false, []() {});
+  if (swept && lt < ND) {
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+      w_out[((size_t)cell * NF + f) * ND + lt] = double(L.a[lc][f][q]);
+  }
+}
 
 // u (n_cells cells) <- u + M^-1 A(w_in); w_out <- CK(u) over [0, dt] about 0.
 // w_in and w_out must differ; u is read and written in place.
 template <int DIM, int K, typename Number>
 __global__ void __launch_bounds__((AderFusedShape<DIM, K>::BLOCK))
     ader_sweep_ck_kernel(const DevMesh mesh, const double *__restrict__ w_in, double *u,
-                         const double *__restrict__ cktab, const CkTab ckt, double dt,
-                         double *__restrict__ w_out) {
+                         double dt, double *__restrict__ w_out) {
   using F = AderFusedShape<DIM, K>;
   using S = Shape<DIM, K>;
-  using CS = CkShape<K>;
-  constexpr int ND = S::ND, NF = S::NF, CPB = F::CPB, LOW = F::LOW;
+  constexpr int ND = S::ND, NF = S::NF, CPB = F::CPB, LANES = F::LANES;
   // the sweep's LDS, then (after a barrier) the CK's in the same bytes
   // (3D k=4: 16 KB, 10 groups per CU)
   __shared__ union {
     CartLds<DIM, K, Number> sweep;
-    struct {
-      Number a[CPB][NF][ND];
-      Number b[CPB][NF][ND];
-      Number c[CPB][NF][LOW];
-      Number tab[CS::TAB_SIZE];
-    } ck;
+    AderFusedCk<DIM, K, Number, CPB> ck;
   } lds;
 
   const int tid = threadIdx.x;
@@ -78,7 +101,7 @@ __global__ void __launch_bounds__((AderFusedShape<DIM, K>::BLOCK))
                             cell, swept, cscale, bv, k);
   double un[NF];
   if (swept) {
-    const int lane = tid - lc * CartShape<DIM, K>::LANES;
+    const int lane = tid - lc * LANES;
     const double ea1 = epi.a1 * cscale;
     const size_t cbase = (size_t)cell * NF * ND;
 #pragma unroll
@@ -88,26 +111,12 @@ __global__ void __launch_bounds__((AderFusedShape<DIM, K>::BLOCK))
     }
   }
   __syncthreads();  // every lane is done with the sweep's LDS
-  // the CK tables (visible after ck_cell's first barrier)
-  for (int i = tid; i < CS::TAB_SIZE && i < ckt.size; i += blockDim.x)
-    lds.ck.tab[i] = Number(cktab[i]);
-
-  // ---- the CK of step n+1 on the same cells (ader_ck_kernel's set-up) ----
-  const int lck = tid / ND;
-  const int q = tid - lck * ND;
-  const bool lane_ok = lck < CPB;
-  const int lcc = lane_ok ? lck : 0;
-  // the same cells on the same lanes: a node lane of the CK is a swept lane
-  const bool active = lane_ok && swept;
-  Number rho_inv, rc2, ih[DIM];
-  ck_factors<DIM, true>(mesh, cell, active, rho_inv, rc2, ih);
-  Number uc[NF];
-#pragma unroll
-  for (int f = 0; f < NF; ++f) uc[f] = active ? Number(un[f]) : Number(0);
-  ck_cell<DIM, K, Number, true>(mesh, nullptr, lds.ck.tab, ckt, dt, 0.0, 0.0, lds.ck.a, lds.ck.b,
-                                lds.ck.c, nullptr, lck, lcc, q, lane_ok, active,
-                                (size_t)(active ? cell : 0) * NF * ND, rho_inv, rc2, ih, uc,
-                                w_out);
+  // the CK of step n+1 on the same cells (a slot past the last cell computes on
+  // some cell and stores nothing)
+  const int slot = tid / LANES;
+  const int e = xcd_remap(blockIdx.x, gridDim.x) * CPB + slot;
+  fused_ck<DIM, K, Number, CPB>(lds.ck, mesh, min(e, mesh.n_cells - 1), slot, tid - slot * LANES,
+                                e < mesh.n_cells, un, dt, w_out);
 }
 
 // The same fusion with the sweep half in the gathered-trace form of
@@ -118,11 +127,12 @@ __global__ void __launch_bounds__((AderFusedShape<DIM, K>::BLOCK))
 // points straight from the neighbours' nodes in memory, instead of the
 // neighbours' fields being staged in LDS.  The LDS of the sweep shrinks to the
 // cell's fields and the lines' dp/dt shares (3D k=4: 7.4 KB; the union is then
-// the CK's 9.4 KB instead of 16 KB) and the registers to 68 (k=4), so a CU
-// holds 14 groups instead of 10 for the CK's latency-bound phases: 3D k=4 64^3
-// 90.1 -> 97.9, k=5 40^3 71.8 -> 84.0, k=3 64^3 115 -> 127 GDoF/s per ADER
-// step (FP64).  The FP32
-// operator keeps the staged form (117 against 107 GDoF/s at k=4).
+// the CK's 7 KB instead of 16 KB): 3D k=4 64^3 90.1 -> 97.9, k=5 40^3 71.8 -> 84.0,
+// k=3 64^3 115 -> 127 GDoF/s per ADER step (FP64, with the CK of one lane per node).
+// With the CK in line form (ader_ck_lines_kernel's), on another card: k=4 94.0 ->
+// 102.3, k=3 126.7 -> 131.2, FP32 k=4 113.4 -> 118.4, k=3 138.4 -> 140.4 GDoF/s; the sweep half's memory
+// latency and the VALU (5.3e8 instructions at k=4) share the time at 12 groups per
+// CU.  The FP32 operator keeps the staged form.
 // The arithmetic is dg_operator_cart_kernel's expression for expression (the
 // traces' chains over the same values, the line phase in the three passes of
 // dg_operator_cartg_kernel, the pressure shares summed in the same order): the
@@ -135,20 +145,20 @@ struct AderFusedGShape {
   // each cell on whole waves, with a lane for each of its nodes and lines
   static constexpr bool ENABLED = DIM == 3 && K >= 3 && K <= 5 && CPB * LANES == BLOCK &&
                                   LANES % 64 == 0 && ND <= LANES && NLINE <= LANES;
+  // k=4: 82 -> 80 registers, 12 groups per CU instead of 10; k=5: 99 -> 92, 5 groups
+  // instead of 4 (7 waves would spill 43 registers at k=4)
+  static constexpr int MIN_WAVES = K == 4 ? 6 : K == 5 ? 5 : 1;
 };
 
 // u (n_cells cells, CPB per group) <- u + M^-1 A(w_in); w_out <- CK(u) over
 // [0, dt] about 0.  w_in and w_out must differ; u is read and written in place.
 template <int DIM, int K, typename Number>
-__global__ void __launch_bounds__((AderFusedGShape<DIM, K>::BLOCK))
+__global__ void __launch_bounds__((AderFusedGShape<DIM, K>::BLOCK), (AderFusedGShape<DIM, K>::MIN_WAVES))
     ader_sweepg_ck_kernel(const DevMesh mesh, const double *__restrict__ w_in, double *u,
-                          const double *__restrict__ cktab, const CkTab ckt, double dt,
-                          double *__restrict__ w_out) {
+                          double dt, double *__restrict__ w_out) {
   using F = AderFusedGShape<DIM, K>;
-  using CS = CkShape<K>;
   constexpr int N = F::N, ND = F::ND, NT = F::NT, NF = F::NF, NFACE = 2 * DIM;
   constexpr int NLINE = F::NLINE, CPB = F::CPB, LANES = F::LANES;
-  constexpr int LOW = AderFusedShape<DIM, K>::LOW;
   constexpr const CartConst<N> &T = CartTable<N>::value;
   __shared__ __align__(16) union {
     struct {
@@ -157,12 +167,7 @@ __global__ void __launch_bounds__((AderFusedGShape<DIM, K>::BLOCK))
       Number fc[CPB][NFACE][8];
       Number vc[CPB][DIM][2];
     } sw;
-    struct {
-      Number a[CPB][NF][ND];
-      Number b[CPB][NF][ND];
-      Number c[CPB][NF][LOW];
-      Number tab[CS::TAB_SIZE];
-    } ck;
+    AderFusedCk<DIM, K, Number, CPB> ck;
   } lds;
 
   // the lane's cell slot (uniform over a wave) and its lane within the cell;
@@ -361,25 +366,7 @@ __global__ void __launch_bounds__((AderFusedGShape<DIM, K>::BLOCK))
     }
   }
   __syncthreads();  // every lane is done with the sweep's LDS
-  // ---- the CK of step n+1 on the same cell (ader_sweep_ck_kernel's) ----
-  for (int i = tid; i < CS::TAB_SIZE && i < ckt.size; i += blockDim.x)
-    lds.ck.tab[i] = Number(cktab[i]);
-  // the CK's lanes: node q of cell slot lck, the sweep's node lane of the same
-  // cell (ND = LANES at 3D k=3; one cell per group at k=4, 5)
-  const int lck = tid / ND;
-  const int q = tid - lck * ND;
-  const bool lane_ok = lck < CPB;
-  const int lcc = lane_ok ? lck : 0;
-  const bool active = lane_ok && swept;
-  Number rho_inv, rc2, ih[DIM];
-  ck_factors<DIM, true>(mesh, cell, active, rho_inv, rc2, ih);
-  Number uc[NF];
-#pragma unroll
-  for (int f = 0; f < NF; ++f) uc[f] = active ? Number(un[f]) : Number(0);
-  ck_cell<DIM, K, Number, true>(mesh, nullptr, lds.ck.tab, ckt, dt, 0.0, 0.0, lds.ck.a, lds.ck.b,
-                                lds.ck.c, nullptr, lck, lcc, q, lane_ok, active,
-                                (size_t)(active ? cell : 0) * NF * ND, rho_inv, rc2, ih, uc,
-                                w_out);
+  fused_ck<DIM, K, Number, CPB>(lds.ck, mesh, cell, lc, lt, swept, un, dt, w_out);
 }
 
 }  // namespace exw

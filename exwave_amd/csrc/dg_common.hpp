@@ -111,6 +111,22 @@ __device__ __forceinline__ int xcd_remap(int b, int nblk) {
   return x * q + (x < r ? x : r) + i;
 }
 
+// x / D and x % D of a lane's small index, 0 <= x < 4096: full-rate 24-bit
+// products (the compiler's division by a constant takes 32-bit high products at
+// a quarter of the rate).  Exact: with M = ceil(2^S / D), x (M D - 2^S) < 2^S.
+template <int D>
+__device__ __forceinline__ int small_div(int x) {
+  if constexpr (D == 1) return x;
+  constexpr int S = D >= 16 ? 24 : 20;
+  constexpr unsigned M = ((1u << S) + D - 1) / D;
+  static_assert(D <= 4096, "the quotient of 12-bit indices");
+  return int(__umul24(unsigned(x), M) >> S);
+}
+template <int D>
+__device__ __forceinline__ int small_mod(int x) {
+  return x - __mul24(small_div<D>(x), D);
+}
+
 template <int N>
 __device__ __forceinline__ constexpr int pow_n(int e) {
   return e == 0 ? 1 : (e == 1 ? N : N * N);

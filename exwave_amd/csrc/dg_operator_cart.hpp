@@ -375,7 +375,9 @@ __global__ void __launch_bounds__((CartLines<DIM, K, Number>::BLOCK))
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int dir = wave / WPD;
   const int li = tid - dir * (WPD * 64);
-  const int lcB = CPB == 1 ? 0 : li / NT, t = li - lcB * NT, t0 = t % N, t1 = t / N;
+  static_assert(NF * ND <= 4096 && NPP * BLOCK <= 4096, "small_div's range");
+  const int lcB = CPB == 1 ? 0 : small_div<NT>(li), t = li - lcB * NT, t0 = small_mod<N>(t),
+            t1 = small_div<N>(t);
   const bool line_ok = dir < DIM && (CPB == 1 ? t < NT : lcB < CPB);
   auto line_base = [&](auto D_) __attribute__((always_inline)) {
     constexpr int d = decltype(D_)::value;
@@ -407,11 +409,11 @@ __global__ void __launch_bounds__((CartLines<DIM, K, Number>::BLOCK))
   int dst[NPP];     // and in s_u; -1: none
 #pragma unroll
   for (int j = 0; j < NPP; ++j) {
-    const int p = tid + j * BLOCK, lc = CPB == 1 ? 0 : min(p / PPC, CPB - 1);
+    const int p = tid + j * BLOCK, lc = CPB == 1 ? 0 : min(small_div<PPC>(p), CPB - 1);
     int e = 2 * (p - lc * PPC);
     const bool ok = e < NF * ND;
     if (!ok || ((NF * ND) % 2 && e == NF * ND - 1)) e = NF * ND - 2;  // (the odd last pair overlaps)
-    dst[j] = ok ? lc * (NF * NDP) + e / N * NX + e % N : -1;
+    dst[j] = ok ? lc * (NF * NDP) + (NX == N ? e : e + small_div<N>(e)) : -1;
     idx[j] = (size_t)cell_of(lc) * (NF * ND) + e;
     __builtin_memcpy(&own[j], src + idx[j], 16);
   }
@@ -421,7 +423,7 @@ __global__ void __launch_bounds__((CartLines<DIM, K, Number>::BLOCK))
   auto load_faces = [&](int d) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < NPF; ++j) {
-      const int q = tid + j * BLOCK, g = min(q / PPF, 4 * CPB - 1);  // field g of the round
+      const int q = tid + j * BLOCK, g = min(small_div<PPF>(q), 4 * CPB - 1);  // field g of the round
       const int lc = g / 4, s = (g >> 1) & 1, c = g & 1;
       int e = 2 * min(q - g * PPF, PPF - 1);
       if (ND % 2 && e == ND - 1) e = ND - 2;
@@ -433,11 +435,11 @@ __global__ void __launch_bounds__((CartLines<DIM, K, Number>::BLOCK))
   auto put_faces = [&](int d) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < NPF; ++j) {
-      const int q = tid + j * BLOCK, g = q / PPF;
+      const int q = tid + j * BLOCK, g = small_div<PPF>(q);
       int e = 2 * (q - g * PPF);
       if (ND % 2 && e == ND - 1) e = ND - 2;
       if (g < 4 * CPB) {
-        Number *o = &s_nb[(FULL ? 4 * d : 0) + (g & 3)][g >> 2][e / N * NX + e % N];
+        Number *o = &s_nb[(FULL ? 4 * d : 0) + (g & 3)][g >> 2][NX == N ? e : e + small_div<N>(e)];
         o[0] = Number(nbv[d][j].x);
         o[1] = Number(nbv[d][j].y);
       }
@@ -584,7 +586,7 @@ __global__ void __launch_bounds__((CartLines<DIM, K, Number>::BLOCK))
   };
 #pragma unroll
   for (int j = 0; j < NPP; ++j) {
-    const int p = tid + j * BLOCK, lc = CPB == 1 ? 0 : min(p / PPC, CPB - 1);
+    const int p = tid + j * BLOCK, lc = CPB == 1 ? 0 : min(small_div<PPC>(p), CPB - 1);
     if (dst[j] < 0 || (CPB > 1 && c0 + lc >= n_entries)) continue;
     const double cscale = epi.cell_scale ? epi.cell_scale[cell_of(lc)] : 1.0;
     if (cscale == 0.0) continue;

@@ -176,7 +176,9 @@ __global__ void __launch_bounds__((GenShape<DIM, K>::BLOCK))
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int dir = wave / WPD;
   const int li = tid - dir * (WPD * 64);
-  const int lcB = CPB == 1 ? 0 : li / NT, t = li - lcB * NT, t0 = t % N, t1 = t / N;
+  static_assert(NF * ND <= 4096 && NPP * BLOCK <= 4096, "small_div's range");
+  const int lcB = CPB == 1 ? 0 : small_div<NT>(li), t = li - lcB * NT, t0 = small_mod<N>(t),
+            t1 = small_div<N>(t);
   const bool line_ok = dir < DIM && (CPB == 1 ? t < NT : lcB < CPB);
   // f(direction) at compile time, for the waves that hold lines
   auto lines = [&](auto f) __attribute__((always_inline)) {
@@ -228,12 +230,12 @@ __global__ void __launch_bounds__((GenShape<DIM, K>::BLOCK))
   int dst[NPP];  // the pair's place in a [CPB][NF][NDP] LDS array; -1: none
 #pragma unroll
   for (int j = 0; j < NPP; ++j) {
-    const int p = tid + j * BLOCK, lc = CPB == 1 ? 0 : min(p / PPC, CPB - 1);
+    const int p = tid + j * BLOCK, lc = CPB == 1 ? 0 : min(small_div<PPC>(p), CPB - 1);
     int e = 2 * (p - lc * PPC);
     const bool ok = e < NF * ND;
     if (!ok) e = NF * ND - 2;
     if ((NF * ND) % 2 && e == NF * ND - 1) e = NF * ND - 2;  // (the last pair overlaps)
-    dst[j] = ok ? lc * (NF * NDP) + e / N * NX + e % N : -1;
+    dst[j] = ok ? lc * (NF * NDP) + (NX == N ? e : e + small_div<N>(e)) : -1;
     const int cell = cell_of(lc);
     const double *uc = src + (size_t)cell * (NF * ND) + e;
 #pragma unroll
@@ -452,9 +454,10 @@ __global__ void __launch_bounds__((GenShape<DIM, K>::BLOCK))
   Number kv[NPL][DIM], jxw[NPL];
 #pragma unroll
   for (int j = 0; j < NPL; ++j) {
-    const int n = tid + j * BLOCK, lc = CPB == 1 ? 0 : n / ND, q = n - lc * ND;
-    const int qi[3] = {q % N, (q / N) % N, DIM == 3 ? q / (N * N) : 0};
-    const int ql = q / N * NX + q % N;
+    const int n = tid + j * BLOCK, lc = CPB == 1 ? 0 : small_div<ND>(n), q = n - lc * ND;
+    const int r = small_div<N>(q), qi[3] = {q - r * N, DIM == 3 ? small_mod<N>(r) : r,
+                                             DIM == 3 ? small_div<N>(r) : 0};
+    const int ql = NX == N ? q : q + r;
     if (n >= NODES) continue;
     const int cell = cell_of(lc);
     const Number rho = Number(mesh.rho[cell]), cc = Number(mesh.speed[cell]);
@@ -524,9 +527,10 @@ __global__ void __launch_bounds__((GenShape<DIM, K>::BLOCK))
   // ---------------- E: nodes ----------------
 #pragma unroll
   for (int j = 0; j < NPL; ++j) {
-    const int n = tid + j * BLOCK, lc = CPB == 1 ? 0 : n / ND, q = n - lc * ND;
-    const int qi[3] = {q % N, (q / N) % N, DIM == 3 ? q / (N * N) : 0};
-    const int ql = q / N * NX + q % N;
+    const int n = tid + j * BLOCK, lc = CPB == 1 ? 0 : small_div<ND>(n), q = n - lc * ND;
+    const int r = small_div<N>(q), qi[3] = {q - r * N, DIM == 3 ? small_mod<N>(r) : r,
+                                             DIM == 3 ? small_div<N>(r) : 0};
+    const int ql = NX == N ? q : q + r;
     if (n >= NODES) continue;
     Number fv[DIM], kp = Number(0);
 #pragma unroll
@@ -554,7 +558,7 @@ __global__ void __launch_bounds__((GenShape<DIM, K>::BLOCK))
   // ---------------- epilogue, pairs of entries ----------------
 #pragma unroll
   for (int j = 0; j < NPP; ++j) {
-    const int p = tid + j * BLOCK, lc = CPB == 1 ? 0 : min(p / PPC, CPB - 1);
+    const int p = tid + j * BLOCK, lc = CPB == 1 ? 0 : min(small_div<PPC>(p), CPB - 1);
     if (dst[j] < 0 || (CPB > 1 && c0 + lc >= mesh.n_cells)) continue;
     const double cscale = epi.cell_scale ? epi.cell_scale[c0 + lc] : 1.0;
     if (cscale == 0.0) continue;

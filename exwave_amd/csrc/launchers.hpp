@@ -58,9 +58,9 @@ using PostErrLaunch = hipError_t (*)(const DevMesh &, const double *, const DevM
 
 // (mesh, first cell, cell count, per-cell flux coefficients out, stream)
 using CoefLaunch = hipError_t (*)(const DevMesh &, int, int, double *, hipStream_t);
-// (mesh, w_in, u (in place), CK table, CK offsets, dt, w_out, stream)
-using AderFusedLaunch = hipError_t (*)(const DevMesh &, const double *, double *, const double *,
-                                       const CkTab &, double, double *, hipStream_t);
+// (mesh, w_in, u (in place), dt, w_out, stream)
+using AderFusedLaunch = hipError_t (*)(const DevMesh &, const double *, double *, double, double *,
+                                       hipStream_t);
 
 struct DimKernels {
   CoefLaunch coef;
@@ -186,22 +186,22 @@ hipError_t launch_op(const DevMesh &m, const double *src, const double *tab,
 }
 
 template <int DIM, int K, typename Number>
-hipError_t launch_ader_fused(const DevMesh &m, const double *w_in, double *u, const double *cktab,
-                             const CkTab &ck, double dt, double *w_out, hipStream_t s) {
+hipError_t launch_ader_fused(const DevMesh &m, const double *w_in, double *u, double dt,
+                             double *w_out, hipStream_t s) {
   if constexpr (AderFusedGShape<DIM, K>::ENABLED && std::is_same_v<Number, double>) {
     // gathered neighbour traces (FP64, 3D k = 3..5)
     using G = AderFusedGShape<DIM, K>;
     const int grid = (m.n_cells + G::CPB - 1) / G::CPB;
     if (grid == 0) return hipSuccess;
     hipLaunchKernelGGL((ader_sweepg_ck_kernel<DIM, K, Number>), dim3(grid),
-                       dim3(AderFusedGShape<DIM, K>::BLOCK), 0, s, m, w_in, u, cktab, ck, dt, w_out);
+                       dim3(AderFusedGShape<DIM, K>::BLOCK), 0, s, m, w_in, u, dt, w_out);
     return hipGetLastError();
   }
   using F = AderFusedShape<DIM, K>;
   const int grid = (m.n_cells + F::CPB - 1) / F::CPB;
   if (grid == 0) return hipSuccess;
   hipLaunchKernelGGL((ader_sweep_ck_kernel<DIM, K, Number>), dim3(grid), dim3(F::BLOCK), 0, s, m,
-                     w_in, u, cktab, ck, dt, w_out);
+                     w_in, u, dt, w_out);
   return hipGetLastError();
 }
 
@@ -221,14 +221,19 @@ template <int DIM, int K, typename Number, bool CART>
 hipError_t launch_ck(const DevMesh &m, const double *src, const double *recon,
                      const double *cktab, const CkTab &ck, double t2, double t1, double te,
                      const CellSel *sel, double *out, hipStream_t s) {
-  using G = CkGroup<DIM, K>;
   CellSel cs{};
   if (sel) cs = *sel;
   const int n = cs.list ? cs.n : m.n_cells;
-  const int grid = (n + G::CPB - 1) / G::CPB;
-  if (grid == 0) return hipSuccess;
-  hipLaunchKernelGGL((ader_ck_kernel<DIM, K, Number, CART>), dim3(grid), dim3(G::BLOCK), 0, s,
-                     m, src, recon, cktab, ck, t2, t1, te, cs, out);
+  if (n == 0) return hipSuccess;
+  if constexpr (CART) {
+    using G = CkLinesShape<DIM, K>;
+    hipLaunchKernelGGL((ader_ck_lines_kernel<DIM, K, Number>), dim3((n + G::CPB - 1) / G::CPB),
+                       dim3(G::BLOCK), 0, s, m, src, recon, t2, t1, te, cs, out);
+  } else {
+    using G = CkGroup<DIM, K>;
+    hipLaunchKernelGGL((ader_ck_kernel<DIM, K, Number>), dim3((n + G::CPB - 1) / G::CPB),
+                       dim3(G::BLOCK), 0, s, m, src, recon, cktab, ck, t2, t1, te, cs, out);
+  }
   return hipGetLastError();
 }
 

@@ -1,0 +1,49 @@
+"""The Cauchy-Kowalevski integral on box cells (ader_ck_lines_kernel: one lane per
+line, whole waves per direction) against the oracle: cells with a different size in
+each direction, varying media, groups that hold several cells with the last one
+part-filled, odd numbers of entries per cell, vectors that start on an odd 8 bytes,
+with and without the given first derivative, on an interval away from its
+expansion time; nothing outside the output's cells is written."""
+import numpy as np
+import pytest
+
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dim,k,nint", [
+    (2, 1, 5), (2, 2, 5), (2, 3, 3), (2, 4, 5), (2, 5, 3), (2, 7, 3), (2, 9, 3), (2, 11, 2),
+    (2, 12, 3), (3, 1, 3), (3, 2, 3), (3, 3, 3), (3, 4, 2), (3, 5, 2), (3, 6, 2), (3, 9, 2)])
+def test_ck_lines_vs_oracle(dim, k, nint):
+    import torch
+
+    import exwave_amd as X
+    print("ck lines", dim, k, nint, flush=True)
+    om = O.Mesh(dim, nint, 0, 0, 0.0, 2)
+    V = np.ctypeslib.as_array(om._m.contents.vertices, shape=(om.n_cells, 1 << dim, dim))
+    V *= np.array([1.0, 0.6, 1.7][:dim])
+    rng = np.random.default_rng(41)
+    om.set_material(rng.uniform(0.5, 2.0, om.n_cells), rng.uniform(0.5, 2.0, om.n_cells))
+    op = X.WaveOperator(X.Context(0), dim, k, om.vertices, om.neighbor, om.rho, om.speed)
+    assert op.is_cartesian
+    N = om.n_dofs(k)
+    u, rec = rng.standard_normal(N), rng.standard_normal(N)
+    t2, t1, te = 0.011, 0.004, 0.002
+
+    def dev(a, off):
+        t = torch.zeros(N + 4, dtype=torch.float64, device="cuda")
+        t[off:off + N] = torch.from_numpy(a)
+        return t[off:off + N]
+
+    for off in (0, 1):
+        for r in (None, rec):
+            want = om.ader_ck(k, u, r, t2, t1, te)
+            full = torch.full((N + 4,), 7.0, dtype=torch.float64, device="cuda")
+            op.ader_ck(dev(u, off), None if r is None else dev(r, 1 - off), t2, t1, te,
+                       full[off + 1:off + 1 + N])
+            got = full.cpu().numpy()
+            # a value is a chain of at most some hundred roundings over terms of the
+            # size of the largest entries: far below 1e-12 of the maximum
+            assert np.max(np.abs(got[off + 1:off + 1 + N] - want)) <= 1e-12 * np.max(np.abs(want))
+            assert np.all(got[:off + 1] == 7.0) and np.all(got[off + 1 + N:] == 7.0)
