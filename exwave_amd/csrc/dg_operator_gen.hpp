@@ -53,7 +53,9 @@ namespace exw {
 // filled line waves), twice as many 12-60 % (fewer groups per CU); 3D k=6 lost
 // 40 % with 384 instead of its three line waves, 3D k=8 the same with six waves
 // instead of eight (two groups per CU: unevenly spread over the SIMDs).
-template <int DIM, int K>
+// SMALL: a wave's worth of nodes per group instead of a wave of lines per direction,
+// for launches of few groups (GenSmall).
+template <int DIM, int K, bool SMALL = false>
 struct GenShape {
   static constexpr int N = K + 1;
   static constexpr int ND = DIM == 2 ? N * N : N * N * N;
@@ -61,7 +63,7 @@ struct GenShape {
   static constexpr int NF = DIM + 1;
   static constexpr int NFACE = 2 * DIM;
   static constexpr int WPD = (NT + 63) / 64;
-  static constexpr int CPB = NT >= 64 ? 1 : 64 / NT;
+  static constexpr int CPB = SMALL ? (ND >= 64 ? 1 : 64 / ND) : (NT >= 64 ? 1 : 64 / NT);
   static constexpr int LINE_LANES = DIM * WPD * 64;
   static constexpr int NODES = CPB * ND;
   // nodes beyond the line waves get waves of their own up to 256 lanes (512 for
@@ -69,7 +71,7 @@ struct GenShape {
   // few-lane tasks, which outnumber its nodes (3D 113 -> 93 us, 60^3 cells)
   static constexpr int NODE_CAP = ND >= 512 ? 512 : 256;
   static constexpr int NODE_LANES =
-      NODES >= NODE_CAP || K == 1 ? NODE_CAP : (NODES + 63) / 64 * 64;
+      NODES >= NODE_CAP || (K == 1 && !SMALL) ? NODE_CAP : (NODES + 63) / 64 * 64;
   static constexpr int BLOCK = K == 6 && DIM == 3 ? LINE_LANES
                                : LINE_LANES > NODE_LANES ? LINE_LANES : NODE_LANES;
   static constexpr int NPL = (NODES + BLOCK - 1) / BLOCK;
@@ -83,6 +85,20 @@ struct GenShape {
   // waves per SIMD to hold the registers to, one or two below the compiler's
   // own choice (no spills)
   static constexpr int MIN_WAVES = DIM == 3 ? (K <= 5 ? 5 : 4) : (K <= 3 ? 6 : 4);
+};
+
+// Whether a launch over n cells runs the small groups: while the full ones are few
+// its time is that of one group from start to end, which a smaller one finishes
+// earlier; with more cells the small groups' emptier lanes cost more.  2D, ten
+// launches in us, small against full groups: k=4 506 cells (43 full groups) 54.0
+// against 64.8, k=5 361 cells (37) 56 against 71, k=7 196 cells (25) 65 against 77;
+// near 230 full groups the small ones take 77, 82 and 100, the full ones about what
+// they take above: the lines cross at 102 to 157 full groups.
+template <int DIM, int K>
+struct GenSmall {
+  static constexpr bool EXISTS =
+      (DIM == 2 ? K >= 3 : K >= 2) && GenShape<DIM, K>::CPB > GenShape<DIM, K, true>::CPB;
+  static bool pays(int n) { return EXISTS && n < 128 * GenShape<DIM, K>::CPB; }
 };
 
 // Jinv[e*DIM+i] = dxi_e/dx_i of J; returns det J (as multilinear_jacobian)
@@ -127,12 +143,12 @@ __device__ __forceinline__ float recip_sqrt(float x) {
   return __builtin_fmaf(0.5f * y, __builtin_fmaf(-x * y, y, 1.0f), y);
 }
 
-template <int DIM, int K, typename Number>
-__global__ void __launch_bounds__((GenShape<DIM, K>::BLOCK))
-    __attribute__((amdgpu_waves_per_eu(GenShape<DIM, K>::MIN_WAVES)))
+template <int DIM, int K, typename Number, bool SMALL = false>
+__global__ void __launch_bounds__((GenShape<DIM, K, SMALL>::BLOCK))
+    __attribute__((amdgpu_waves_per_eu(GenShape<DIM, K, SMALL>::MIN_WAVES)))
     dg_operator_gen_kernel(const DevMesh mesh, const double *__restrict__ src,
                            const Epilogue epi) {
-  using S = GenShape<DIM, K>;
+  using S = GenShape<DIM, K, SMALL>;
   constexpr int N = S::N, ND = S::ND, NT = S::NT, NF = S::NF, NFACE = S::NFACE;
   constexpr int BLOCK = S::BLOCK, CPB = S::CPB, NX = S::NX, NDP = S::NDP, NV = 1 << DIM;
   constexpr int WPD = S::WPD, NPL = S::NPL, NODES = S::NODES;

@@ -177,6 +177,15 @@ hipError_t launch_op(const DevMesh &m, const double *src, const double *tab,
   } else {
     using G = GenShape<DIM, K>;
     if (e.cell_list) return hipErrorInvalidValue;  // cell lists: Cartesian kernel only
+    if constexpr (GenSmall<DIM, K>::EXISTS)
+      if (GenSmall<DIM, K>::pays(m.n_cells)) {
+        using H = GenShape<DIM, K, true>;
+        const int grid = (m.n_cells + H::CPB - 1) / H::CPB;
+        if (grid == 0) return hipSuccess;
+        hipLaunchKernelGGL((dg_operator_gen_kernel<DIM, K, Number, true>), dim3(grid),
+                           dim3(H::BLOCK), 0, s, m, src, e);
+        return hipGetLastError();
+      }
     const int grid = (m.n_cells + G::CPB - 1) / G::CPB;
     if (grid == 0) return hipSuccess;
     hipLaunchKernelGGL((dg_operator_gen_kernel<DIM, K, Number>), dim3(grid), dim3(G::BLOCK), 0, s,
