@@ -92,8 +92,8 @@ struct GenShape {
 // earlier; with more cells the small groups' emptier lanes cost more.  2D, ten
 // launches in us, small against full groups: k=4 506 cells (43 full groups) 54.0
 // against 64.8, k=5 361 cells (37) 56 against 71, k=7 196 cells (25) 65 against 77;
-// near 230 full groups the small ones take 77, 82 and 100, the full ones about what
-// they take above: the lines cross at 102 to 157 full groups.
+// near 230 full groups the small ones take 77, 82 and 100, the full ones 68, 76 and
+// 83: the lines cross between 100 and 160 full groups.
 template <int DIM, int K>
 struct GenSmall {
   static constexpr bool EXISTS =
