@@ -20,7 +20,8 @@ CSRC = os.path.join(HERE, "csrc")
 OUT_DIR = os.path.join(HERE, "_lib")
 LIB = os.path.join(OUT_DIR, "libexwave_amd.so")
 ARCH = os.environ.get("EXWAVE_ARCH", "gfx950")
-SOURCES = ["kernels_2d.hip", "kernels_3d.hip", "exwave_capi.hip", "exwave_driver.hip", "exwave_serving.hip",
+SOURCES = ["kernels_2d_k11_12.hip", "kernels_3d_k5_7.hip", "kernels_2d_k9_10.hip", "kernels_2d_k6_8.hip",
+           "kernels_3d_k8_12.hip", "kernels_3d_k1_4.hip", "kernels_2d_k1_5.hip", "kernels.hip", "exwave_capi.hip", "exwave_driver.hip", "exwave_serving.hip",
            "exwave_lts.hip", "exwave_output.hip", "exwave_adapt.hip"]
 
 

@@ -335,10 +335,10 @@ hipError_t launch_post_error(const DevMesh &m, const double *tab, const DevModes
   return hipGetLastError();
 }
 
-template <int DIM, int K>
+// the entries of degrees LOW..K
+template <int DIM, int K, int LOW>
 void fill_dim_kernels(DimKernels &t) {
-  t.coef = launch_cart_coef<DIM>;
-  if constexpr (K >= 1 && Shape<DIM, K>::ND > 1024) {
+  if constexpr (K >= LOW && Shape<DIM, K>::ND > 1024) {
     // more nodes than lanes: the operator (any geometry and precision), the
     // projection and the norms; CK, LTS, hanging faces, the error estimator
     // and the post-processing stay unsupported
@@ -352,8 +352,8 @@ void fill_dim_kernels(DimKernels &t) {
     t.block[K] = BigShape<DIM, K>::BLOCK;
     t.cells_per_block[K] = 1;
     t.pipe[K] = false;
-    fill_dim_kernels<DIM, K - 1>(t);
-  } else if constexpr (K >= 1) {
+    fill_dim_kernels<DIM, K - 1, LOW>(t);
+  } else if constexpr (K >= LOW) {
     t.op[K][0][0] = launch_op<DIM, K, double, false>;
     t.op[K][0][1] = launch_op<DIM, K, double, true>;
     t.op[K][1][0] = launch_op<DIM, K, float, false>;
@@ -378,9 +378,19 @@ void fill_dim_kernels(DimKernels &t) {
     t.block[K] = Shape<DIM, K>::BLOCK;
     t.cells_per_block[K] = Shape<DIM, K>::CPB;
     t.pipe[K] = PipeShape<DIM, K>::ENABLED && (DIM == 2 || K <= 5);
-    fill_dim_kernels<DIM, K - 1>(t);
+    fill_dim_kernels<DIM, K - 1, LOW>(t);
   }
 }
+
+// the translation units of the degrees (each compiles by itself: a dimension in
+// one piece takes minutes)
+void fill_2d_k1_5(DimKernels &t);
+void fill_2d_k6_8(DimKernels &t);
+void fill_2d_k9_10(DimKernels &t);
+void fill_2d_k11_12(DimKernels &t);
+void fill_3d_k1_4(DimKernels &t);
+void fill_3d_k5_7(DimKernels &t);
+void fill_3d_k8_12(DimKernels &t);
 
 const DimKernels &kernels_2d();
 const DimKernels &kernels_3d();
