@@ -443,8 +443,10 @@ __device__ __forceinline__ void column_sum(double *v, int idx, int first, double
 // eigenvectors SV (SV^T W SV = 1), so z = SV3 (1 / sum_e g_e lambda) SV3^T r,
 // the constant left out.  On box cells that is the exact inverse (one
 // iteration); on the deformed membranes 8-14 iterations reach the 1e-13 that
-// plain CG needs 60-150 for.  The stop is on r.z, the energy norm of the
-// error in that metric.
+// plain CG needs 60-150 for.  The relative stop is on r.z, the energy norm of the
+// error in that metric; the absolute one on |r| at the Gauss points.  A cell
+// whose p.Ap is at the bottom of the exponent range (a state that has decayed
+// to 1e-150) ends with what it has: the ratio of two such numbers is noise.
 //
 // Lanes hold columns: every tensor is P registers per lane along the last
 // direction, a pass along it is register FMAs, and the other directions
@@ -688,6 +690,17 @@ __global__ void __launch_bounds__((PostColumns<DIM, K>::BLOCK))
     post::column_sum<LPC, BLOCK, 1>(v, idx, lc * LPC, s_red);
     return v[0];
   };
+  // r.z and r.r
+  auto residual = [&](const double *r, const double *z, double (&v)[2]) {
+    v[0] = v[1] = 0.0;
+#pragma unroll
+    for (int j = 0; j < P; ++j) {
+      v[0] += r[j] * z[j];
+      v[1] += r[j] * r[j];
+    }
+    if (!act) v[0] = v[1] = 0.0;
+    post::column_sum<LPC, BLOCK, 2>(v, idx, lc * LPC, s_red);
+  };
 
   double u[P], r[P], p[P];
   div(val, r);  // (val[0..DIM-1] holds the right-hand side's flux)
@@ -695,7 +708,8 @@ __global__ void __launch_bounds__((PostColumns<DIM, K>::BLOCK))
   for (int j = 0; j < P; ++j) u[j] = 0.0;
   precond(r, p);
   double rz = dot(r, p);
-  const double stop = cfg.rel_tol * cfg.rel_tol * rz;
+  const double stop = cfg.rel_tol * cfg.rel_tol * rz, stop_abs = cfg.abs_tol * cfg.abs_tol;
+  const double guard = fmax(1e-5 * stop_abs, 1e4 * 2.2250738585072014e-308);  // as plain CG's
   // a zero right-hand side (or NaN) leaves u = 0 (or NaN, through r)
   bool done = !(rz > 0.0);
   if (done && !(rz == 0.0)) u[0] = rz - rz;
@@ -705,7 +719,7 @@ __global__ void __launch_bounds__((PostColumns<DIM, K>::BLOCK))
     laplace(p, q);
     const double pAp = dot(p, q);
     if (!done) {
-      const double alpha = rz / pAp;
+      const double alpha = pAp < guard ? 0.0 : rz / pAp;
 #pragma unroll
       for (int j = 0; j < P; ++j) {
         u[j] += alpha * p[j];
@@ -713,11 +727,12 @@ __global__ void __launch_bounds__((PostColumns<DIM, K>::BLOCK))
       }
     }
     precond(r, q);
-    const double rn = dot(r, q);
+    double rn[2];
+    residual(r, q, rn);
     if (!done) {
-      const double beta = rn / rz;
-      rz = rn;
-      done = !(rn > stop);
+      const double beta = rn[0] / rz;
+      rz = rn[0];
+      done = pAp < guard || !(rn[0] > stop) || rn[1] < stop_abs;
 #pragma unroll
       for (int j = 0; j < P; ++j) p[j] = q[j] + beta * p[j];
     }

@@ -67,6 +67,29 @@ def test_post_pcg(X, case):
     assert torch.isnan(post[: (k + 2) ** dim]).all()
 
 
+@pytest.mark.parametrize("dim,nint,k", [(2, 10, 3), (2, 10, 4), (3, 4, 2), (3, 3, 4)])
+def test_post_pcg_scales(X, dim, nint, k):
+    """States that have decayed: down to the bottom of the exponent range every cell
+    ends finite and of the state's size (p* is linear in the state while the
+    residuals are above EXW_POST_ABS_TOL; below it p* may fall back to the average,
+    and products of two residuals underflow from 1e-154 on)."""
+    import torch
+    print("post scales", dim, nint, k, flush=True)
+    om, op, u = _setup(X, dim, nint, O.TRANSFORM_AXIS_2PI, 0.06, k)
+    src = torch.from_numpy(u).cuda()
+    tmp = torch.zeros_like(src)
+    one, post = (torch.zeros(op.n_post, dtype=torch.float64, device="cuda") for _ in range(2))
+    op.post_pressure(src, tmp, one)
+    top = float(one.abs().max())
+    for e in [3, 20, 100] + list(range(138, 172)) + [200, 290]:
+        s = 10.0 ** -e
+        op.post_pressure(src * s, tmp, post)
+        assert torch.isfinite(post).all(), e
+        assert float(post.abs().max()) <= 4 * top * s, e
+        if e == 3:
+            assert float((post - s * one).abs().max()) <= 1e-10 * top * s
+
+
 @pytest.mark.parametrize("dim,nint,k", [(2, 5, 1), (2, 3, 6), (2, 2, 12), (3, 3, 1), (3, 3, 4),
                                         (3, 2, 7), (3, 2, 8), (3, 2, 9), (3, 1, 12)])
 def test_l2_errors_edges(X, dim, nint, k):
