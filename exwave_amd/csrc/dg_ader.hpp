@@ -552,8 +552,8 @@ __device__ __forceinline__ void ck_lines(Number *a, Number *b, bool ok, int d, i
     get(N0{}, v, p);
 #pragma unroll
     for (int i = 0; i < N; ++i) {
-      cv[0][i] = c0 * v[i];
-      cp[0][i] = c0 * p[i];
+      cv[0][i] = v[i];
+      cp[0][i] = p[i];
     }
   }
   // the first derivative: u' = -derive(u), or the given one; carried negated
@@ -572,11 +572,12 @@ __device__ __forceinline__ void ck_lines(Number *a, Number *b, bool ok, int d, i
   } else {
     derive(N0{}, b);
   }
+  // (the leading term's product in the FMA: one rounding of its size)
   if (ok)
 #pragma unroll
     for (int i = 0; i < N; ++i) {
-      cv[0][i] = fma_of(-c1, v[i], cv[0][i]);
-      cp[0][i] = fma_of(-c1, p[i], cp[0][i]);
+      cv[0][i] = fma_of(c0, cv[0][i], -c1 * v[i]);
+      cp[0][i] = fma_of(c0, cp[0][i], -c1 * p[i]);
     }
 
   double fac = -0.5, p2 = a2 * a2, p1 = a1 * a1;
@@ -679,10 +680,14 @@ __device__ __forceinline__ void ck_lines(Number *a, Number *b, bool ok, int d, i
         Number x[NLO];
 #pragma unroll
         for (int i = 0; i < NLO; ++i) x[i] = a[f * LD + o + i * st];
+        // (summed by itself: one rounding of the larger terms' size)
 #pragma unroll
-        for (int i = 0; i < NHI; ++i)
+        for (int i = 0; i < NHI; ++i) {
+          Number y = Number(L.V[i * NLO]) * x[0];
 #pragma unroll
-          for (int m = 0; m < NLO; ++m) c[i] = fma_of(Number(L.V[i * NLO + m]), x[m], c[i]);
+          for (int m = 1; m < NLO; ++m) y = fma_of(Number(L.V[i * NLO + m]), x[m], y);
+          c[i] += y;
+        }
       };
       add(d, cv[LV - 1]);
       if (d == 0) add(DIM, cp[LV - 1]);

@@ -47,3 +47,39 @@ def test_ck_lines_vs_oracle(dim, k, nint):
             # size of the largest entries: far below 1e-12 of the maximum
             assert np.max(np.abs(got[off + 1:off + 1 + N] - want)) <= 1e-12 * np.max(np.abs(want))
             assert np.all(got[:off + 1] == 7.0) and np.all(got[off + 1 + N:] == 7.0)
+
+
+@pytest.mark.parametrize("dim,k,n", [(2, 1, 100), (2, 4, 60), (2, 7, 70), (3, 2, 16), (3, 4, 13),
+                                     (3, 6, 11)])
+def test_ck_lines_fp32_roundings(dim, k, n):
+    """The FP32 operator rounds the integral's leading term no more often than the
+    kernel of general cells, which runs the same mesh as soon as one vertex is off
+    the grid: once when the state is read and once per term that is added.  With
+    terms of a few thousandths of each other three roundings count (the third
+    derivative's term is below the last bit), a fourth would raise the root mean
+    square of the relative error by sqrt(4 / 3) = 1.155: the line is at sqrt(3.5 / 3),
+    some tens of standard errors of the 10^5 values from both."""
+    import torch
+
+    import exwave_amd as X
+    print("ck roundings", dim, k, n, flush=True)
+    ctx = X.Context(0)
+    V, nb = X.mesh_hypercube(dim, n)
+    one = np.ones(V.shape[0])
+    W = V.copy()
+    W[-1, -1, 0] += 0.1 / n
+    g = torch.Generator(device="cuda").manual_seed(7)
+    rms = []
+    for vertices in (V, W):
+        op = X.WaveOperator(ctx, dim, k, vertices, nb, one, one)
+        assert op.is_cartesian == (vertices is V)
+        r = torch.rand((2, op.n_dofs), generator=g, dtype=torch.float64, device="cuda")
+        u = torch.exp2(r[0]) * torch.sign(r[1] - 0.5)
+        want, got = op.new_vector(), op.new_vector()
+        dt = 2e-3 / (n * k * k)
+        op.ader_ck(u, None, dt, 0.0, 0.0, want, X.FP64)
+        op.ader_ck(u, None, dt, 0.0, 0.0, got, X.FP32)
+        rel = ((got - want) / want).view(V.shape[0], -1)[:-1]
+        rms.append(float(rel.square().mean().sqrt()))
+    print("rms", rms)
+    assert rms[0] <= (3.5 / 3) ** 0.5 * rms[1]
