@@ -10,10 +10,12 @@
 // (source/wave_equation_operations.cc:287-313, 1238-1255), and the
 // lower-degree contributions are interpolated back at the end.
 //
-// GPU layout, general cells: one lane per top-level Gauss node; the working
-// field is double buffered in LDS; the level-0 contribution stays in registers,
-// lower levels' contributions live in LDS.  Box cells: one lane per line, the
-// velocities in registers throughout (ck_lines).
+// GPU layout, node form: one lane per top-level Gauss node; the working field is
+// double buffered in LDS; the level-0 contribution stays in registers, lower
+// levels' contributions live in LDS.  On box cells each derivative runs in line
+// form (one lane per line of the level, then one per node) where that was
+// measured faster.  Line form, large launches of box cells: one lane per line
+// throughout, the velocities in registers (ck_lines; CkLinesFrom draws the line).
 #pragma once
 #include <type_traits>
 #include <utility>
@@ -59,16 +61,26 @@ struct CkShape {
   }();
 };
 
-// Cells per workgroup of the general CK kernel.  Its barrier-separated passes
-// wait on every wave of the group, so fewer cells per group pay: in 3D one cell
-// per group from 100 nodes on, two below; 2D keeps the operator's grouping.
+// Cells per workgroup of the CK kernel.  Its 18 barrier-separated passes per
+// cell wait on every wave of the group, so fewer cells per group pay: in 3D
+// one cell per group from 100 nodes on (k=4, 64^3: 1.041 against 1.117 ms
+// with two), two below (k=3: 0.315 against 0.323 ms with four); 2D keeps the
+// operator's grouping.
 template <int DIM, int K>
 struct CkGroup {
   static constexpr int ND = Shape<DIM, K>::ND;
   static constexpr int MAXC = DIM == 3 ? (ND >= 100 ? 1 : 2) : 16;
   static constexpr int CPB = Shape<DIM, K>::CPB < MAXC ? Shape<DIM, K>::CPB : MAXC;
   static constexpr int BLOCK = ((CPB * ND + 63) / 64) * 64;
+  // 3D k=6 sits one register above 6 waves per SIMD (81 VGPRs): held to 6 it
+  // spills 2 and runs 0.633 against 0.735 ms at 32^3 (FP64); elsewhere no hint
+  static constexpr int MIN_WAVES = (DIM == 3 && K == 6) ? 6 : 1;
 };
+
+template <int DIM, int N>
+__device__ __forceinline__ constexpr int ipow_c() {
+  return DIM == 2 ? N * N : N * N * N;
+}
 
 namespace ck {
 
@@ -76,44 +88,135 @@ using exw::static_for;
 
 // Physical derivative at node qq of a level field of NN points per direction
 // (in[f][...] in LDS): outv_d = rho^-1 d_d p, outp = rho c^2 div v (the
-// time derivative is minus this).
-template <int DIM, int NN, int LD, typename Number>
+// time derivative is minus this).  Cartesian: d_d = (1/h_d) d/dxi_d.
+template <int DIM, int NN, int LD, bool CART, typename Number>
 __device__ __forceinline__ void derive(const Number (*in)[LD], const Number *Dl, const Number *Xl,
-                                       int qq, Number rho_inv, Number rc2, const double *V,
-                                       Number *outv, Number &outp) {
+                                       int qq, const Number *ih, Number rho_inv, Number rc2,
+                                       const double *V, Number *outv, Number &outp) {
   const int qd[3] = {qq % NN, (qq / NN) % NN, DIM == 3 ? qq / (NN * NN) : 0};
   constexpr int st[3] = {1, NN, NN * NN};
-  Number gr[DIM + 1][DIM];
+  if constexpr (CART) {
+    Number div = Number(0);
 #pragma unroll
-  for (int e = 0; e < DIM; ++e) {
-    const int q0 = qq - qd[e] * st[e];
-    Number dr[NN];
+    for (int d = 0; d < DIM; ++d) {
+      const int q0 = qq - qd[d] * st[d];
+      const Number *Dr = Dl + qd[d] * NN;
+      Number gp = Number(0), gv = Number(0);
 #pragma unroll
-    for (int m = 0; m < NN; ++m) dr[m] = Dl[qd[e] * NN + m];
-#pragma unroll
-    for (int f = 0; f <= DIM; ++f) {
-      Number g = Number(0);
-#pragma unroll
-      for (int m = 0; m < NN; ++m) g += dr[m] * in[f][q0 + m * st[e]];
-      gr[f][e] = g;
+      for (int m = 0; m < NN; ++m) {
+        const Number dm = Dr[m];
+        gp += dm * in[DIM][q0 + m * st[d]];
+        gv += dm * in[d][q0 + m * st[d]];
+      }
+      outv[d] = rho_inv * gp * ih[d];
+      div += gv * ih[d];
     }
-  }
-  Number xi[DIM], J[DIM * DIM], Ji[DIM * DIM];
+    outp = rc2 * div;
+  } else {
+    Number gr[DIM + 1][DIM];
 #pragma unroll
-  for (int d = 0; d < DIM; ++d) xi[d] = Xl[qd[d]];
-  multilinear_jacobian<DIM>(V, xi, J, Ji);
+    for (int e = 0; e < DIM; ++e) {
+      const int q0 = qq - qd[e] * st[e];
+      Number dr[NN];
+#pragma unroll
+      for (int m = 0; m < NN; ++m) dr[m] = Dl[qd[e] * NN + m];
+#pragma unroll
+      for (int f = 0; f <= DIM; ++f) {
+        Number g = Number(0);
+#pragma unroll
+        for (int m = 0; m < NN; ++m) g += dr[m] * in[f][q0 + m * st[e]];
+        gr[f][e] = g;
+      }
+    }
+    Number xi[DIM], J[DIM * DIM], Ji[DIM * DIM];
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) xi[d] = Xl[qd[d]];
+    multilinear_jacobian<DIM>(V, xi, J, Ji);
+    Number div = Number(0);
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) {
+      Number pg = Number(0);
+#pragma unroll
+      for (int e = 0; e < DIM; ++e) {
+        pg += gr[DIM][e] * Ji[e * DIM + d];
+        div += gr[d][e] * Ji[e * DIM + d];
+      }
+      outv[d] = rho_inv * pg;
+    }
+    outp = rc2 * div;
+  }
+}
+
+// The same Cartesian derivative in line form, for lane `line` < DIM * NN^(DIM-1)
+// of a cell: along its line (direction d) the lane reads p and v_d of `in` into
+// registers once and, at the line's nodes, writes rho^-1 (d/dxi_d p) into
+// out[d] and d/dxi_d v_d over in[d] (only this lane reads those entries of
+// in[d]); derive_nodes then applies 1/h and forms the divergence.  The 1D
+// matrix is the compile-time one of NN Gauss points (CartTable, built by the
+// same routines as the level's table), and every sum and product runs in
+// derive's order: N reads per line instead of N per node and direction.
+template <int DIM, int NN, int LD, typename Number>
+__device__ __forceinline__ void derive_line(Number (*in)[LD], Number (*out)[LD], int line,
+                                            Number rho_inv) {
+  constexpr int NT = DIM == 2 ? NN : NN * NN;
+  constexpr const CartConst<NN> &T = CartTable<NN>::value;
+  const int d = line / NT, t = line - d * NT;
+  int base, sd;
+  if constexpr (DIM == 2) {
+    base = d == 0 ? t * NN : t;
+    sd = d == 0 ? 1 : NN;
+  } else {
+    const int t0 = t % NN, t1 = t / NN;
+    base = d == 0 ? t0 * NN + t1 * NN * NN : (d == 1 ? t0 + t1 * NN * NN : t0 + t1 * NN);
+    sd = d == 0 ? 1 : (d == 1 ? NN : NN * NN);
+  }
+  Number pl[NN], vl[NN];
+#pragma unroll
+  for (int m = 0; m < NN; ++m) {
+    pl[m] = in[DIM][base + m * sd];
+    vl[m] = in[d][base + m * sd];
+  }
+#pragma unroll
+  for (int i = 0; i < NN; ++i) {
+    Number gp = Number(0), gv = Number(0);
+#pragma unroll
+    for (int m = 0; m < NN; ++m) {
+      const Number dm = Number(T.D[i * NN + m]);
+      gp += dm * pl[m];
+      gv += dm * vl[m];
+    }
+    out[d][base + i * sd] = rho_inv * gp;
+    in[d][base + i * sd] = gv;
+  }
+}
+
+// The node half of the line form (after a barrier): outv_d = (rho^-1 d/dxi_d p)
+// / h_d from out[d], and outp = rho c^2 sum_d (d/dxi_d v_d) / h_d from in[d].
+template <int DIM, int LD, typename Number>
+__device__ __forceinline__ void derive_nodes(const Number (*in)[LD], const Number (*out)[LD],
+                                             int qq, const Number *ih, Number rc2, Number *outv,
+                                             Number &outp) {
   Number div = Number(0);
 #pragma unroll
   for (int d = 0; d < DIM; ++d) {
-    Number pg = Number(0);
-#pragma unroll
-    for (int e = 0; e < DIM; ++e) {
-      pg += gr[DIM][e] * Ji[e * DIM + d];
-      div += gr[d][e] * Ji[e * DIM + d];
-    }
-    outv[d] = rho_inv * pg;
+    outv[d] = out[d][qq] * ih[d];
+    div += in[d][qq] * ih[d];
   }
   outp = rc2 * div;
+}
+
+// whether the lines of a level of NN points fit the cell's lanes
+template <int DIM, int NN, int ND>
+constexpr bool lines_fit() {
+  return DIM * (DIM == 2 ? NN : NN * NN) <= ND;
+}
+
+// where the line form was measured faster (CK kernel alone): FP64 everywhere
+// (3D k=4: 1.11 against 1.31 ms at 64^3, k=6: 0.66 against 0.93 ms at 32^3,
+// 3D k=3 equal); FP32 only in 3D from k=4 (at 3D k=3 and 2D it lost 8-10 %)
+template <int DIM, int K, typename Number>
+constexpr bool derive_lines_pay() {
+  return std::is_same_v<Number, double> || (DIM == 3 && K >= 4);
 }
 
 // One tensor pass along direction DIR of the matrix M (NO x NI, row-major) on
@@ -173,11 +276,32 @@ __device__ __forceinline__ bool pass_reg(const Number *M, const Number (*in)[LDI
 
 }  // namespace ck
 
-// The Cauchy-Kowalevski work of the group's cells (general geometry, one lane
-// per node) once the lane's node value u of its cell is known (in registers):
-// the Taylor levels in LDS, the time integral over [t1, t2] about te written to
-// tempsrc.
-template <int DIM, int K, typename Number>
+// The cell's factors of the CK derivatives: 1/rho, rho c^2 and (Cartesian)
+// 1/h_d; 1 for lanes without a cell.  Reciprocals by the hardware estimate
+// and two Newton steps (recip), not IEEE divisions: every lane computes them.
+template <int DIM, bool CART, typename Number>
+__device__ __forceinline__ void ck_factors(const DevMesh &mesh, int cell, bool active,
+                                           Number &rho_inv, Number &rc2, Number (&ih)[DIM]) {
+  Number rho = Number(1), cc = Number(1);
+#pragma unroll
+  for (int d = 0; d < DIM; ++d) ih[d] = Number(1);
+  if (active) {
+    rho = Number(mesh.rho[cell]);
+    cc = Number(mesh.speed[cell]);
+    if constexpr (CART) {
+#pragma unroll
+      for (int d = 0; d < DIM; ++d) ih[d] = recip(Number(mesh.h[(size_t)cell * DIM + d]));
+    }
+  }
+  rho_inv = recip(rho);
+  rc2 = rho * cc * cc;
+}
+
+// The Cauchy-Kowalevski work of the group's cells once the lane's node value
+// u of its cell is known (in registers): the Taylor levels in LDS, the time
+// integral over [t1, t2] about te written to tempsrc.  Shared by
+// ader_ck_kernel and the fused ADER sweep, so both give the same bits.
+template <int DIM, int K, typename Number, bool CART>
 __device__ __forceinline__ void ck_cell(
     const DevMesh &mesh, const double *__restrict__ recon, const Number *s_ck, const CkTab &ckt,
     double t2, double t1, double te, Number (*s_a)[Shape<DIM, K>::NF][Shape<DIM, K>::ND],
@@ -187,7 +311,7 @@ __device__ __forceinline__ void ck_cell(
                       ? CkShape<K>::low_off(DIM, CkShape<K>::N_LEVELS)
                       : 1],
     const double *Vc, int lc, int lcc, int q, bool lane_ok, bool active, size_t cbase,
-    Number rho_inv, Number rc2, const Number (&u)[Shape<DIM, K>::NF],
+    Number rho_inv, Number rc2, const Number (&ih)[DIM], const Number (&u)[Shape<DIM, K>::NF],
     double *__restrict__ tempsrc) {
   using S = Shape<DIM, K>;
   using CS = CkShape<K>;
@@ -209,15 +333,26 @@ __device__ __forceinline__ void ck_cell(
     for (int f = 0; f < NF; ++f) up[f] = active ? Number(recon[cbase + f * ND + q]) : Number(0);
   } else {
     Number ov[DIM], op;
-    ck::derive<DIM, N, ND>(s_a[lcc], s_ck + ckt.off_D[0], s_ck + ckt.off_X[0], q, rho_inv, rc2, Vc,
-                           ov, op);
+    if constexpr (CART && ck::lines_fit<DIM, N, ND>() && ck::derive_lines_pay<DIM, K, Number>()) {
+      if (lane_ok && q < DIM * (DIM == 2 ? N : N * N))
+        ck::derive_line<DIM, N, ND>(s_a[lc], s_b[lc], q, rho_inv);
+      __syncthreads();
+      ck::derive_nodes<DIM, ND>(s_a[lcc], s_b[lcc], q, ih, rc2, ov, op);
+    } else {
+      ck::derive<DIM, N, ND, CART>(s_a[lcc], s_ck + ckt.off_D[0], s_ck + ckt.off_X[0], q, ih,
+                                   rho_inv, rc2, Vc, ov, op);
+    }
 #pragma unroll
     for (int d = 0; d < DIM; ++d) up[d] = -ov[d];
     up[DIM] = -op;
   }
 #pragma unroll
   for (int f = 0; f < NF; ++f) contrib[f] = Number(a2 - a1) * u[f] + c1 * up[f];
-  __syncthreads();  // (the derivative reads other nodes' entries of s_a)
+  // the node form of the derivative reads other nodes' entries of s_a: wait
+  // for every lane before overwriting; the line form's node half (and the
+  // reconstruction input) read only the lane's own entries
+  if constexpr (!(CART && ck::lines_fit<DIM, N, ND>() && ck::derive_lines_pay<DIM, K, Number>()))
+    __syncthreads();
   if (lane_ok) {
 #pragma unroll
     for (int f = 0; f < NF; ++f) s_a[lc][f][q] = -up[f];
@@ -238,11 +373,21 @@ __device__ __forceinline__ void ck_cell(
     const Number fac_t = Number(fac * (p2 - p1));
     Number(*cur)[ND] = parity ? s_b[lcc] : s_a[lcc];
     Number(*nxt)[ND] = parity ? s_a[lcc] : s_b[lcc];
+    constexpr bool LINES = CART && ck::lines_fit<DIM, n, ND>() && ck::derive_lines_pay<DIM, K, Number>();
+    if constexpr (LINES) {
+      if (lane_ok && q < DIM * (DIM == 2 ? n : n * n))
+        ck::derive_line<DIM, n, ND>(cur, nxt, q, rho_inv);
+      __syncthreads();
+    }
     if (q < nd) {
       Number ov[DIM], op;
-      ck::derive<DIM, n, ND>(cur, s_ck + ckt.off_D[LEVEL], s_ck + ckt.off_X[LEVEL], q, rho_inv, rc2,
-                             Vc, ov, op);
+      if constexpr (LINES)
+        ck::derive_nodes<DIM, ND>(cur, nxt, q, ih, rc2, ov, op);
+      else
+        ck::derive<DIM, n, ND, CART>(cur, s_ck + ckt.off_D[LEVEL], s_ck + ckt.off_X[LEVEL], q,
+                                     ih, rho_inv, rc2, Vc, ov, op);
       if (lane_ok) {
+        // (the line phase left rho^-1 d/dxi_d p there: this lane's own entries)
 #pragma unroll
         for (int d = 0; d < DIM; ++d) nxt[d][q] = ov[d];
         nxt[DIM][q] = op;
@@ -332,8 +477,9 @@ __device__ __forceinline__ void ck_cell(
   }
 }
 
-template <int DIM, int K, typename Number>
+template <int DIM, int K, typename Number, bool CART>
 __global__ void __launch_bounds__((CkGroup<DIM, K>::BLOCK))
+    __attribute__((amdgpu_waves_per_eu(CkGroup<DIM, K>::MIN_WAVES)))
     ader_ck_kernel(const DevMesh mesh, const double *__restrict__ src,
                    const double *__restrict__ recon, const double *__restrict__ cktab,
                    const CkTab ckt, double t2, double t1, double te_all, const CellSel sel,
@@ -348,7 +494,7 @@ __global__ void __launch_bounds__((CkGroup<DIM, K>::BLOCK))
   __shared__ Number s_a[CPB][NF][ND];
   __shared__ Number s_b[CPB][NF][ND];
   __shared__ Number s_c[CPB][NF][LOW];
-  __shared__ double s_V[CPB][(1 << DIM) * DIM];
+  __shared__ double s_V[CART ? 1 : CPB][CART ? 1 : (1 << DIM) * DIM];
   __shared__ Number s_ck[CS::TAB_SIZE];
 
   const int tid = threadIdx.x;
@@ -363,16 +509,17 @@ __global__ void __launch_bounds__((CkGroup<DIM, K>::BLOCK))
   const bool active = lane_ok && cell >= 0 && cell < mesh.n_cells;
   const double te = active && sel.cluster ? sel.te[sel.cluster[cell]] : te_all;
 
-  constexpr int NVD = (1 << DIM) * DIM;
-  for (int i = tid; i < CPB * NVD; i += blockDim.x) {
-    const int c2 = cell_of(blockIdx.x * CPB + i / NVD);
-    s_V[i / NVD][i % NVD] =
-        c2 >= 0 && c2 < mesh.n_cells ? mesh.vertices[(size_t)c2 * NVD + i % NVD] : 0.0;
+  if constexpr (!CART) {
+    constexpr int NVD = (1 << DIM) * DIM;
+    for (int i = tid; i < CPB * NVD; i += blockDim.x) {
+      const int c2 = cell_of(blockIdx.x * CPB + i / NVD);
+      s_V[i / NVD][i % NVD] =
+          c2 >= 0 && c2 < mesh.n_cells ? mesh.vertices[(size_t)c2 * NVD + i % NVD] : 0.0;
+    }
   }
-  const Number rho = Number(active ? mesh.rho[cell] : 1.0),
-               cc = Number(active ? mesh.speed[cell] : 1.0);
-  const Number rho_inv = recip(rho), rc2 = rho * cc * cc;
-  const double *Vc = s_V[lcc];
+  Number rho_inv, rc2, ih[DIM];
+  ck_factors<DIM, CART>(mesh, cell, active, rho_inv, rc2, ih);
+  const double *Vc = CART ? nullptr : s_V[CART ? 0 : lcc];
 
   const size_t cbase = (size_t)cell * NF * ND;
   Number u[NF];
@@ -382,11 +529,53 @@ __global__ void __launch_bounds__((CkGroup<DIM, K>::BLOCK))
 #pragma unroll
     for (int f = 0; f < NF; ++f) u[f] = Number(src[cbase + f * ND + q]);
   }
-  ck_cell<DIM, K, Number>(mesh, recon, s_ck, ckt, t2, t1, te, s_a, s_b, s_c, Vc, lc, lcc, q, lane_ok,
-                          active, cbase, rho_inv, rc2, u, tempsrc);
+  ck_cell<DIM, K, Number, CART>(mesh, recon, s_ck, ckt, t2, t1, te, s_a, s_b, s_c, Vc, lc, lcc,
+                                q, lane_ok, active, cbase, rho_inv, rc2, ih, u, tempsrc);
 }
 
 // ---------------------------------------------------------------------------
+// From how many groups of the node form (CkGroup) on a launch over box cells runs
+// the line form; 1 << 30: never.  The line form's matrices are constants of its
+// unrolled code, 10 to 100 KB of it that every launch fetches once: a launch that
+// leaves most of the chip idle waits for the instructions (2D k=7, 100 cells, FP32:
+// 13.0 us against 6.6, k=12 38.7 against 14.2), and at 2D k=12 the code does not
+// stay in the instruction cache at all (FP32 47524 cells: 802 us against 515).  The
+// node form reads its matrices from LDS in short loops.  us, node form / line form:
+//   FP64 2D k=4   256 cells 5.9 / 6.1,  3969 6.9 / 6.6;  k=6 841 9.5 / 9.9,
+//        2025 11.6 / 10.1, 54289 135 / 58
+//        2D k=8  1225 16.4 / 17.4,  2304 20.6 / 19.7;  k=10 1521 28.4 / 31.1,
+//        2704 47 / 32;  k=11 676 22.5 / 34.3, 1296 39.7 / 35
+//        3D k=4   216 6.4 / 6.8, 1000 8.2 / 7.9;  k=6 216 11.4 / 11.8, 343
+//        14.2 / 13.2;  k=7 216 14.4 / 15.5, 512 19.8 / 17.9
+//   FP32 2D k=4  3969 6.0 / 6.7,  13225 9.6 / 7.9;  k=6 3721 9.7 / 11.5, 6724
+//        15 / 11.9;  k=7 2916 9.8 / 13.7, 5184 16.3 / 14.3;  k=9 6724 38.7 / 39.8,
+//        26569 132 / 106;  k=10 5476 45.6 / 50.3, 66049 446 / 337;  k=11 2304
+//        26.6 / 32.4, 4624 48.9 / 33.7
+//        3D k=4  1000 7.2 / 7.8, 2197 10.5 / 10.0;  k=6 729 14.0 / 15.2, 1331
+//        22.9 / 20.6;  k=7 512 15.5 / 17.1, 1000 26.8 / 20.1
+// Never: 3D k=5 (lines fill 36 of a wave's 64 lanes: 4913 cells 38.9 / 41.8), k=8, 9
+// (two waves per direction, registers: 592 / 632 at k=9, 5832 cells), 2D k=12, and
+// FP32 k=3 (2D 83521 cells 13.0 / 14.1, 3D 15625 13.0 / 15.1).
+template <int DIM, int K, typename Number>
+struct CkLinesFrom {
+  static constexpr int NEVER = 1 << 30;
+  static constexpr bool D = std::is_same_v<Number, double>;
+  static constexpr int groups() {
+    if constexpr (DIM == 2) {
+      if (D) return K <= 3 || K == 5 ? 0 : K <= 7 ? 320 : K <= 10 ? 1024 : K == 11 ? 1280 : NEVER;
+      return K <= 2 ? 0 : K == 3 ? NEVER : K <= 5 ? 1024 : K <= 8 ? 1280 : K <= 10 ? 8192
+             : K == 11 ? 3584 : NEVER;
+    } else {
+      if (D) return K <= 2 ? 0 : K == 3 ? 128 : K == 4 ? 512 : K == 6 || K == 7 ? 384 : NEVER;
+      return K <= 2 ? 0 : K == 4 ? 1792 : K == 6 ? 1280 : K == 7 ? 768 : NEVER;
+    }
+  }
+  static constexpr bool ALWAYS = groups() == 0, EXISTS = groups() < NEVER;
+  static bool pays(int n_cells) {
+    return ALWAYS || (EXISTS && n_cells / CkGroup<DIM, K>::CPB >= groups());
+  }
+};
+
 // The Cauchy-Kowalevski work of box cells in line form.  Lane (d, t) of a cell
 // owns line t of direction d.  On a box v_d is only ever differentiated along d
 // and only ever receives d/dxi_d p, so v_d and its Taylor contribution live in

@@ -38,44 +38,74 @@ struct AderFusedShape {
 
 // The CK half of the fused kernels: LDS and the work of the group's cells once
 // node lane lt < ND of cell slot lc holds the new state un (swept: the slot's
-// cell exists).  LANES lanes per cell, line lanes first.
-template <int DIM, int K, typename Number, int CPB>
+// cell exists).  LANES lanes per cell, line lanes first.  LINES: the form that
+// launch_ck picks for the same cells (CkLinesFrom).
+template <int DIM, int K, typename Number, int CPB, bool LINES>
 struct AderFusedCk {
   static constexpr int LD = CkGrid<DIM, K + 1>::SIZE;
   Number a[CPB][DIM + 1][LD];
   Number b[CPB][DIM][LD];
 };
 template <int DIM, int K, typename Number, int CPB>
-__device__ __forceinline__ void fused_ck(AderFusedCk<DIM, K, Number, CPB> &L, const DevMesh &mesh,
-                                         int cell, int lc, int lt, bool swept,
-                                         const double (&un)[DIM + 1], double dt,
-                                         double *__restrict__ w_out) {
+struct AderFusedCk<DIM, K, Number, CPB, false> {
+  static constexpr int NF = DIM + 1, ND = Shape<DIM, K>::ND;
+  static constexpr int LOW = CkShape<K>::low_off(DIM, CkShape<K>::N_LEVELS) > 0
+                                 ? CkShape<K>::low_off(DIM, CkShape<K>::N_LEVELS)
+                                 : 1;
+  Number a[CPB][NF][ND];
+  Number b[CPB][NF][ND];
+  Number c[CPB][NF][LOW];
+  Number tab[CkShape<K>::TAB_SIZE];
+};
+template <int DIM, int K, typename Number, int CPB, bool LINES>
+__device__ __forceinline__ void fused_ck(AderFusedCk<DIM, K, Number, CPB, LINES> &L,
+                                         const DevMesh &mesh, int cell, int lc, int lt, bool swept,
+                                         const double (&un)[DIM + 1],
+                                         const double *__restrict__ cktab, const CkTab &ckt,
+                                         double dt, double *__restrict__ w_out) {
   constexpr int N = K + 1, NT = DIM == 2 ? N : N * N, ND = Shape<DIM, K>::ND, NF = DIM + 1;
-  const int q = CkGrid<DIM, N>::node(lt);
-  if (swept && lt < ND) {
+  if constexpr (LINES) {
+    const int q = CkGrid<DIM, N>::node(lt);
+    if (swept && lt < ND) {
 #pragma unroll
-    for (int f = 0; f < NF; ++f) L.a[lc][f][q] = Number(un[f]);
-  }
-  const bool ok = lt < DIM * NT;
-  const int d = ok ? small_div<NT>(lt) : 0, t = ok ? lt - d * NT : 0;
-  const Number rho = Number(mesh.rho[cell]), cc = Number(mesh.speed[cell]);
-  const Number ih = recip(Number(mesh.h[(size_t)cell * DIM + d]));
-  __syncthreads();
-  ck_lines<DIM, K, Number>(L.a[lc][0], L.b[lc][0], ok, d, t, recip(rho) * ih, (rho * cc * cc) * ih, dt,
-                           0.0, 0.0, false, []() {});
-  if (swept && lt < ND) {
+      for (int f = 0; f < NF; ++f) L.a[lc][f][q] = Number(un[f]);
+    }
+    const bool ok = lt < DIM * NT;
+    const int d = ok ? small_div<NT>(lt) : 0, t = ok ? lt - d * NT : 0;
+    const Number rho = Number(mesh.rho[cell]), cc = Number(mesh.speed[cell]);
+    const Number ih = recip(Number(mesh.h[(size_t)cell * DIM + d]));
+    __syncthreads();
+    ck_lines<DIM, K, Number>(L.a[lc][0], L.b[lc][0], ok, d, t, recip(rho) * ih, (rho * cc * cc) * ih,
+                             dt, 0.0, 0.0, false, []() {});
+    if (swept && lt < ND) {
 #pragma unroll
-    for (int f = 0; f < NF; ++f)
-      w_out[((size_t)cell * NF + f) * ND + lt] = double(L.a[lc][f][q]);
+      for (int f = 0; f < NF; ++f)
+        w_out[((size_t)cell * NF + f) * ND + lt] = double(L.a[lc][f][q]);
+    }
+  } else {
+    // the CK tables (visible after ck_cell's first barrier)
+    for (int i = threadIdx.x; i < CkShape<K>::TAB_SIZE && i < ckt.size; i += blockDim.x)
+      L.tab[i] = Number(cktab[i]);
+    // lanes past the cell's nodes work on the group's first node and store nothing
+    const bool lane_ok = lt < ND, active = lane_ok && swept;
+    Number rho_inv, rc2, ih[DIM], uc[NF];
+    ck_factors<DIM, true>(mesh, cell, active, rho_inv, rc2, ih);
+#pragma unroll
+    for (int f = 0; f < NF; ++f) uc[f] = active ? Number(un[f]) : Number(0);
+    ck_cell<DIM, K, Number, true>(mesh, nullptr, L.tab, ckt, dt, 0.0, 0.0, L.a, L.b, L.c, nullptr,
+                                  lc, lane_ok ? lc : 0, lane_ok ? lt : 0, lane_ok, active,
+                                  (size_t)(active ? cell : 0) * NF * ND, rho_inv, rc2, ih, uc,
+                                  w_out);
   }
 }
 
 // u (n_cells cells) <- u + M^-1 A(w_in); w_out <- CK(u) over [0, dt] about 0.
 // w_in and w_out must differ; u is read and written in place.
-template <int DIM, int K, typename Number>
+template <int DIM, int K, typename Number, bool LINES>
 __global__ void __launch_bounds__((AderFusedShape<DIM, K>::BLOCK))
     ader_sweep_ck_kernel(const DevMesh mesh, const double *__restrict__ w_in, double *u,
-                         double dt, double *__restrict__ w_out) {
+                         const double *__restrict__ cktab, const CkTab ckt, double dt,
+                         double *__restrict__ w_out) {
   using F = AderFusedShape<DIM, K>;
   using S = Shape<DIM, K>;
   constexpr int ND = S::ND, NF = S::NF, CPB = F::CPB, LANES = F::LANES;
@@ -83,7 +113,7 @@ __global__ void __launch_bounds__((AderFusedShape<DIM, K>::BLOCK))
   // (3D k=4: 16 KB, 10 groups per CU)
   __shared__ union {
     CartLds<DIM, K, Number> sweep;
-    AderFusedCk<DIM, K, Number, CPB> ck;
+    AderFusedCk<DIM, K, Number, CPB, LINES> ck;
   } lds;
 
   const int tid = threadIdx.x;
@@ -115,8 +145,8 @@ __global__ void __launch_bounds__((AderFusedShape<DIM, K>::BLOCK))
   // some cell and stores nothing)
   const int slot = tid / LANES;
   const int e = xcd_remap(blockIdx.x, gridDim.x) * CPB + slot;
-  fused_ck<DIM, K, Number, CPB>(lds.ck, mesh, min(e, mesh.n_cells - 1), slot, tid - slot * LANES,
-                                e < mesh.n_cells, un, dt, w_out);
+  fused_ck(lds.ck, mesh, min(e, mesh.n_cells - 1), slot, tid - slot * LANES, e < mesh.n_cells, un,
+           cktab, ckt, dt, w_out);
 }
 
 // The same fusion with the sweep half in the gathered-trace form of
@@ -145,17 +175,17 @@ struct AderFusedGShape {
   // each cell on whole waves, with a lane for each of its nodes and lines
   static constexpr bool ENABLED = DIM == 3 && K >= 3 && K <= 5 && CPB * LANES == BLOCK &&
                                   LANES % 64 == 0 && ND <= LANES && NLINE <= LANES;
-  // k=4: 82 -> 80 registers, 12 groups per CU instead of 10; k=5: 99 -> 92, 5 groups
-  // instead of 4 (7 waves would spill 43 registers at k=4)
-  static constexpr int MIN_WAVES = K == 4 ? 6 : K == 5 ? 5 : 1;
+  // k=4: 82 -> 80 registers, 12 groups per CU instead of 10 (7 waves would spill 43)
+  static constexpr int MIN_WAVES = K == 4 ? 6 : 1;
 };
 
 // u (n_cells cells, CPB per group) <- u + M^-1 A(w_in); w_out <- CK(u) over
 // [0, dt] about 0.  w_in and w_out must differ; u is read and written in place.
-template <int DIM, int K, typename Number>
+template <int DIM, int K, typename Number, bool LINES>
 __global__ void __launch_bounds__((AderFusedGShape<DIM, K>::BLOCK), (AderFusedGShape<DIM, K>::MIN_WAVES))
     ader_sweepg_ck_kernel(const DevMesh mesh, const double *__restrict__ w_in, double *u,
-                          double dt, double *__restrict__ w_out) {
+                          const double *__restrict__ cktab, const CkTab ckt, double dt,
+                          double *__restrict__ w_out) {
   using F = AderFusedGShape<DIM, K>;
   constexpr int N = F::N, ND = F::ND, NT = F::NT, NF = F::NF, NFACE = 2 * DIM;
   constexpr int NLINE = F::NLINE, CPB = F::CPB, LANES = F::LANES;
@@ -167,7 +197,7 @@ __global__ void __launch_bounds__((AderFusedGShape<DIM, K>::BLOCK), (AderFusedGS
       Number fc[CPB][NFACE][8];
       Number vc[CPB][DIM][2];
     } sw;
-    AderFusedCk<DIM, K, Number, CPB> ck;
+    AderFusedCk<DIM, K, Number, CPB, LINES> ck;
   } lds;
 
   // the lane's cell slot (uniform over a wave) and its lane within the cell;
@@ -366,7 +396,7 @@ __global__ void __launch_bounds__((AderFusedGShape<DIM, K>::BLOCK), (AderFusedGS
     }
   }
   __syncthreads();  // every lane is done with the sweep's LDS
-  fused_ck<DIM, K, Number, CPB>(lds.ck, mesh, cell, lc, lt, swept, un, dt, w_out);
+  fused_ck(lds.ck, mesh, cell, lc, lt, swept, un, cktab, ckt, dt, w_out);
 }
 
 }  // namespace exw

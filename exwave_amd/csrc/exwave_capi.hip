@@ -743,7 +743,8 @@ int exw_ader_steps(exw_op op, int n_steps, double dt, double *vec, double *work,
   }
   if ((rc = exw_ader_ck(op, vec, nullptr, dt, 0.0, 0.0, w[0], precision))) return rc;
   for (int s = 1; s < n_steps; ++s)
-    EXW_HIP(fused(op->view(), w[(s - 1) & 1], vec, dt, w[s & 1], op->ctx->stream));
+    EXW_HIP(fused(op->view(), w[(s - 1) & 1], vec, op->d_cktab, op->ck, dt, w[s & 1],
+                  op->ctx->stream));
   return sweep(w[(n_steps - 1) & 1]);
 }
 

@@ -58,9 +58,9 @@ using PostErrLaunch = hipError_t (*)(const DevMesh &, const double *, const DevM
 
 // (mesh, first cell, cell count, per-cell flux coefficients out, stream)
 using CoefLaunch = hipError_t (*)(const DevMesh &, int, int, double *, hipStream_t);
-// (mesh, w_in, u (in place), dt, w_out, stream)
-using AderFusedLaunch = hipError_t (*)(const DevMesh &, const double *, double *, double, double *,
-                                       hipStream_t);
+// (mesh, w_in, u (in place), CK table, CK offsets, dt, w_out, stream)
+using AderFusedLaunch = hipError_t (*)(const DevMesh &, const double *, double *, const double *,
+                                       const CkTab &, double, double *, hipStream_t);
 
 struct DimKernels {
   CoefLaunch coef;
@@ -194,24 +194,37 @@ hipError_t launch_op(const DevMesh &m, const double *src, const double *tab,
   return hipGetLastError();
 }
 
-template <int DIM, int K, typename Number>
-hipError_t launch_ader_fused(const DevMesh &m, const double *w_in, double *u, double dt,
-                             double *w_out, hipStream_t s) {
+template <int DIM, int K, typename Number, bool LINES>
+hipError_t launch_ader_fused_form(const DevMesh &m, const double *w_in, double *u,
+                                  const double *cktab, const CkTab &ck, double dt, double *w_out,
+                                  hipStream_t s) {
   if constexpr (AderFusedGShape<DIM, K>::ENABLED && std::is_same_v<Number, double>) {
     // gathered neighbour traces (FP64, 3D k = 3..5)
     using G = AderFusedGShape<DIM, K>;
     const int grid = (m.n_cells + G::CPB - 1) / G::CPB;
-    if (grid == 0) return hipSuccess;
-    hipLaunchKernelGGL((ader_sweepg_ck_kernel<DIM, K, Number>), dim3(grid),
-                       dim3(AderFusedGShape<DIM, K>::BLOCK), 0, s, m, w_in, u, dt, w_out);
-    return hipGetLastError();
+    hipLaunchKernelGGL((ader_sweepg_ck_kernel<DIM, K, Number, LINES>), dim3(grid), dim3(G::BLOCK),
+                       0, s, m, w_in, u, cktab, ck, dt, w_out);
+  } else {
+    using F = AderFusedShape<DIM, K>;
+    const int grid = (m.n_cells + F::CPB - 1) / F::CPB;
+    hipLaunchKernelGGL((ader_sweep_ck_kernel<DIM, K, Number, LINES>), dim3(grid), dim3(F::BLOCK), 0,
+                       s, m, w_in, u, cktab, ck, dt, w_out);
   }
-  using F = AderFusedShape<DIM, K>;
-  const int grid = (m.n_cells + F::CPB - 1) / F::CPB;
-  if (grid == 0) return hipSuccess;
-  hipLaunchKernelGGL((ader_sweep_ck_kernel<DIM, K, Number>), dim3(grid), dim3(F::BLOCK), 0, s, m,
-                     w_in, u, dt, w_out);
   return hipGetLastError();
+}
+
+// (the CK form of launch_ck for the same cells: the steps agree in every bit)
+template <int DIM, int K, typename Number>
+hipError_t launch_ader_fused(const DevMesh &m, const double *w_in, double *u, const double *cktab,
+                             const CkTab &ck, double dt, double *w_out, hipStream_t s) {
+  using L = CkLinesFrom<DIM, K, Number>;
+  if (m.n_cells == 0) return hipSuccess;
+  if constexpr (L::EXISTS)
+    if (L::pays(m.n_cells))
+      return launch_ader_fused_form<DIM, K, Number, true>(m, w_in, u, cktab, ck, dt, w_out, s);
+  if constexpr (!L::ALWAYS)
+    return launch_ader_fused_form<DIM, K, Number, false>(m, w_in, u, cktab, ck, dt, w_out, s);
+  return hipErrorInvalidValue;
 }
 
 // cells of more nodes than a workgroup has lanes (3D k >= 10), any geometry;
@@ -234,13 +247,17 @@ hipError_t launch_ck(const DevMesh &m, const double *src, const double *recon,
   if (sel) cs = *sel;
   const int n = cs.list ? cs.n : m.n_cells;
   if (n == 0) return hipSuccess;
-  if constexpr (CART) {
-    using G = CkLinesShape<DIM, K>;
-    hipLaunchKernelGGL((ader_ck_lines_kernel<DIM, K, Number>), dim3((n + G::CPB - 1) / G::CPB),
-                       dim3(G::BLOCK), 0, s, m, src, recon, t2, t1, te, cs, out);
-  } else {
+  using L = CkLinesFrom<DIM, K, Number>;
+  if constexpr (CART && L::EXISTS)
+    if (L::pays(n)) {
+      using G = CkLinesShape<DIM, K>;
+      hipLaunchKernelGGL((ader_ck_lines_kernel<DIM, K, Number>), dim3((n + G::CPB - 1) / G::CPB),
+                         dim3(G::BLOCK), 0, s, m, src, recon, t2, t1, te, cs, out);
+      return hipGetLastError();
+    }
+  if constexpr (!(CART && L::ALWAYS)) {
     using G = CkGroup<DIM, K>;
-    hipLaunchKernelGGL((ader_ck_kernel<DIM, K, Number>), dim3((n + G::CPB - 1) / G::CPB),
+    hipLaunchKernelGGL((ader_ck_kernel<DIM, K, Number, CART>), dim3((n + G::CPB - 1) / G::CPB),
                        dim3(G::BLOCK), 0, s, m, src, recon, cktab, ck, t2, t1, te, cs, out);
   }
   return hipGetLastError();

@@ -49,6 +49,41 @@ def test_ck_lines_vs_oracle(dim, k, nint):
             assert np.all(got[:off + 1] == 7.0) and np.all(got[off + 1 + N:] == 7.0)
 
 
+# (the line form runs from a number of cells on that depends on degree and
+# precision: one launch below it and one above, for every degree that has one)
+@pytest.mark.parametrize("dim,k,fp32,below,above", [
+    (2, 4, 0, 50, 57), (2, 6, 0, 39, 41), (2, 7, 0, 35, 37), (2, 8, 0, 55, 56), (2, 9, 0, 45, 46),
+    (2, 10, 0, 45, 46), (2, 11, 0, 35, 36), (3, 3, 0, 6, 7), (3, 4, 0, 7, 8), (3, 6, 0, 7, 8),
+    (3, 7, 0, 7, 8), (2, 4, 1, 100, 102), (2, 5, 1, 84, 86), (2, 6, 1, 79, 81), (2, 7, 1, 71, 73),
+    (2, 8, 1, 61, 63), (2, 9, 1, 127, 129),
+    (3, 4, 1, 12, 13), (3, 6, 1, 10, 11), (3, 7, 1, 9, 10)])
+def test_ck_forms_vs_oracle(dim, k, fp32, below, above):
+    """Both forms around the line between them; intervals of a tenth of h / k^2, so
+    that no term outgrows the state: at most some hundred roundings of the size of
+    the largest entry (1e-12, with the FP32 operator 160 x 2^-24 = 1e-5).  (FP32
+    stops at degree 9: the tenth derivative of random values, which either form
+    holds before the power of the time step scales it, passes 3e38.)"""
+    import torch
+
+    import exwave_amd as X
+    ctx = X.Context(0)
+    for nint in (below, above):
+        print("ck forms", dim, k, fp32, nint, flush=True)
+        om = O.Mesh(dim, nint, 0, 0, 0.0, 2)
+        rng = np.random.default_rng(43)
+        om.set_material(rng.uniform(0.5, 2.0, om.n_cells), rng.uniform(0.5, 2.0, om.n_cells))
+        op = X.WaveOperator(ctx, dim, k, om.vertices, om.neighbor, om.rho, om.speed)
+        u, rec = rng.standard_normal((2, om.n_dofs(k)))
+        s = 0.1 / (nint * k * k)
+        got = op.new_vector()
+        for r in (None, rec * nint):
+            want = om.ader_ck(k, u, r, 1.1 * s, 0.4 * s, 0.2 * s)
+            op.ader_ck(torch.from_numpy(u).cuda(), None if r is None else torch.from_numpy(r).cuda(),
+                       1.1 * s, 0.4 * s, 0.2 * s, got, X.FP32 if fp32 else X.FP64)
+            d = np.max(np.abs(got.cpu().numpy() - want))
+            assert d <= (1e-5 if fp32 else 1e-12) * np.max(np.abs(want))
+
+
 @pytest.mark.parametrize("dim,k,n", [(2, 1, 100), (2, 4, 60), (2, 7, 70), (3, 2, 16), (3, 4, 13),
                                      (3, 6, 11)])
 def test_ck_lines_fp32_roundings(dim, k, n):
