@@ -1,5 +1,6 @@
 // dg_operator_gen.hpp -- fused operator + RK epilogue for general multilinear
-// cells (every degree whose cell fits a workgroup of one lane per node).
+// cells (every degree whose cell fits a workgroup of one lane per node), and the rule
+// by which a launch runs it or a kernel with one lane per node (GenForms).
 //
 // The arithmetic is that of evaluate_cell / evaluate_inner_face /
 // evaluate_boundary_face (source/wave_equation_operations.cc:424-629) on a
@@ -89,16 +90,85 @@ struct GenShape {
 
 // Whether a launch over n cells runs the small groups: while the full ones are few
 // its time is that of one group from start to end, which a smaller one finishes
-// earlier; with more cells the small groups' emptier lanes cost more.  2D, ten
-// launches in us, small against full groups: k=4 506 cells (43 full groups) 54.0
-// against 64.8, k=5 361 cells (37) 56 against 71, k=7 196 cells (25) 65 against 77;
-// near 230 full groups the small ones take 77, 82 and 100, the full ones 68, 76 and
-// 83: the lines cross between 100 and 160 full groups.
+// earlier; with more cells the small groups' emptier lanes cost more.  Degrees whose
+// small launches run this kernel (GenForms).  2D, ten launches in us, small against
+// full groups: k=4 506 cells (43 full groups) 54.0 against 64.8, k=5 361 cells (37)
+// 56 against 71; near 230 full groups the small ones take 77 and 82, the full ones
+// 68 and 76: the lines cross between 100 and 160 full groups.
 template <int DIM, int K>
 struct GenSmall {
-  static constexpr bool EXISTS =
-      (DIM == 2 ? K >= 3 : K >= 2) && GenShape<DIM, K>::CPB > GenShape<DIM, K, true>::CPB;
+  static constexpr bool EXISTS = (DIM == 2 ? K >= 3 && K <= 5 : K >= 2) &&
+                                 GenShape<DIM, K>::CPB > GenShape<DIM, K, true>::CPB;
   static bool pays(int n) { return EXISTS && n < 128 * GenShape<DIM, K>::CPB; }
+};
+
+// Which launches over general cells run the kernels with one lane per node
+// (dg_operator_gen_node_kernel, below 48 nodes dg_operator_kernel) instead of this
+// file's line form: those over from <= n < to cells; `single`: the launch has one
+// output.  The line form's matrices are constants of its unrolled code, which every
+// launch fetches once, and its chain of barriers is longer: small launches wait for
+// both, and at 2D k >= 9 the code leaves the instruction cache.  The node forms read
+// their tables from LDS in short loops.  us per RK stage (two outputs) and, behind
+// the bar, per single-output sweep, node form / line form:
+//   FP64 2D k=1 332929 cells 60 / 50 | 41 / 43;  k=3 11449 8.1 / 8.0 | 5 % lost;  k=4
+//        676 6.1 / 5.5, 1600 6.0 / 6.4, 3969 6.9 / 7.8, 7396 10.9 / 9.4;  k=5 2809 8.8
+//        / 8.7 | 21 % lost, 9216 15.8 / 12.1;  k=6 2025 7.4 / 8.8, 6724 13.5 / 12.4;
+//        k=7 2916 9.2 / 9.6, 5184 12.9 / 11.0;  k=8 2304 10.9 / 11.7, 4096 15.7 /
+//        13.5;  k=9 1849 9.7 / 12.0, 3364 14.6 / 13.6;  k=10 841 7.9 / 12.4, 5476 24.7
+//        / 29.3, 21904 93 / 91 | 71 / 83;  k=11 1296 11.7 / 13.3, 4624 28.0 / 29.5,
+//        18496 107 / 95 | 86 / 84;  k=12 100 6.5 / 14.0, 7921 52.0 / 52.6, 15876 104 /
+//        94 | 82 / 88
+//     3D k=5 343 9.0 / 10.1, 2197 26.0 / 26.2, 4913 55.7 / 51.4 | 27000 220 / 225; k=6
+//       343 10.8 / 11.4, 729 17.1 / 14.4;  k=7 216 10.3 / 12.7, 512 18.9 / 17.1; k=8
+//       729 32.1 / 34.6, 2744 113 / 104 | 101 / 100;  k=9 5832 408 / 412
+//   FP32 2D k=3 11449 6.9 / 7.1 | 6.2 / 6.7;  k=4 1600 5.9 / 6.4, 7396 7.8 / 8.5,
+//        13225 11.7 / 10.2;  k=5 1089 6.1 / 6.5, 5041 8.0 / 8.3, 9216 13.0 / 10.0;
+//        k=6 2025 7.1 / 8.2, 6724 12.9 / 10.4;  k=7 1600 7.0 / 8.0, 5184 12.4 / 10.0;
+//        k=8 2304 8.4 / 14.3, 8281 26.1 / 25.6 | 17 % lost, 32761 96 / 73 | 69 / 66;
+//        k=9 13225 44.1 / 45.2, 26569 86 / 79 | 61 / 71;  k=10 21904 86 / 89, 66049
+//        266 / 257 | 176 / 224;  k=11 9216 49 / 51, 18496 95 / 88 | 73 / 80;  k=12 36
+//        6.1 / 19.8, 47524 281 / 286
+//     3D k=5 729 9.8 / 9.9, 1000 12.1 / 11.2 | 13 % lost, 2197 23.6 / 21.6;  k=6 343
+//       9.6 / 10.3, 729 16.4 / 12.7;  k=7 1728 39 / 41, 4096 86 / 82;  k=8 729 28.7 /
+//       29.7, 1331 50.8 / 49.6;  k=9 216 16.2 / 18.5, 512 29.3 / 27.4
+template <int DIM, int K, typename Number>
+struct GenForms {
+  static constexpr int NEVER = 1 << 30;
+  static constexpr bool D = std::is_same_v<Number, double>;
+  static constexpr int from(bool single) {
+    if constexpr (DIM == 2) {
+      if (K == 1) return D && single ? 30000 : NEVER;
+      if (K == 3) return single ? 6000 : NEVER;
+      if (K == 4) return 1200;
+      if (K == 5) return D && !single ? NEVER : 600;
+      return K >= 6 ? 0 : NEVER;
+    }
+    return K >= 5 ? 0 : NEVER;
+  }
+  static constexpr int to(bool single) {
+    constexpr int f64_2d[13] = {0,    0,    0,    0,    6000,  0,    5500,
+                                4096, 3000, 3000, 12000, 9000, 9000},
+                  f64_2d_single[13] = {0,    NEVER, 0,   32000, 6000,  7500,  5500,
+                                       4096, 3000, 3000, NEVER, 16384, NEVER},
+                  f32_2d[13] = {0,    0,    0,     0,     11000, 7500, 4096,
+                                3584, 8192, 16384, 32768, 12000, NEVER},
+                  f32_2d_single[13] = {0,    0,     0,     0,     11000, 7500, 4096,
+                                       3584, 24000, NEVER, NEVER, NEVER, NEVER},
+                  f64_3d[10] = {0, 0, 0, 0, 0, 2500, 512, 448, 1800, NEVER},
+                  f64_3d_single[10] = {0, 0, 0, 0, 0, NEVER, 512, 448, 2800, NEVER},
+                  f32_3d[10] = {0, 0, 0, 0, 0, 800, 512, 3500, 1152, 448},
+                  f32_3d_single[10] = {0, 0, 0, 0, 0, 2000, 512, 6000, 1152, 448};
+    if constexpr (DIM == 2)
+      return (D ? (single ? f64_2d_single : f64_2d) : (single ? f32_2d_single : f32_2d))[K];
+    else
+      return (D ? (single ? f64_3d_single : f64_3d) : (single ? f32_3d_single : f32_3d))[K];
+  }
+  // (the node form's offsets into the vectors have 32 bits)
+  static bool node(int n, bool single) {
+    return n >= from(single) && n < to(single) &&
+           uint64_t(n) * (GenShape<DIM, K>::NF * GenShape<DIM, K>::ND) < (uint64_t(1) << 32);
+  }
+  static constexpr bool NODE_EXISTS = from(false) < to(false) || from(true) < to(true);
 };
 
 // Jinv[e*DIM+i] = dxi_e/dx_i of J; returns det J (as multilinear_jacobian)

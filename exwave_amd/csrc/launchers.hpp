@@ -9,10 +9,12 @@
 #include "dg_ader_fused.hpp"
 #include "dg_lts.hpp"
 #include "dg_misc.hpp"
+#include "dg_operator.hpp"
 #include "dg_operator_cart.hpp"
 #include "dg_operator_cartg.hpp"
 #include "dg_operator_big.hpp"
 #include "dg_operator_gen.hpp"
+#include "dg_operator_gen_node.hpp"
 #include "dg_operator_pipe.hpp"
 #include "dg_nc.hpp"
 #include "dg_post.hpp"
@@ -87,6 +89,16 @@ struct DimKernels {
 inline bool cart_pipe_enabled() {
   static const bool on = [] {
     const char *v = getenv("EXW_CART_PIPE");
+    return !(v && v[0] == '0');
+  }();
+  return on;
+}
+
+// The kernels of general cells as GenForms chooses them; EXW_GEN_KERNEL=0 selects
+// dg_operator_kernel throughout.
+inline bool gen_kernel_enabled() {
+  static const bool on = [] {
+    const char *v = getenv("EXW_GEN_KERNEL");
     return !(v && v[0] == '0');
   }();
   return on;
@@ -175,21 +187,33 @@ hipError_t launch_op(const DevMesh &m, const double *src, const double *tab,
     hipLaunchKernelGGL((dg_operator_cart_kernel<DIM, K, Number>), dim3(grid), dim3(CS::BLOCK), 0,
                        s, m, src, e);
   } else {
-    using G = GenShape<DIM, K>;
+    using F = GenForms<DIM, K, Number>;
     if (e.cell_list) return hipErrorInvalidValue;  // cell lists: Cartesian kernel only
-    if constexpr (GenSmall<DIM, K>::EXISTS)
-      if (GenSmall<DIM, K>::pays(m.n_cells)) {
-        using H = GenShape<DIM, K, true>;
-        const int grid = (m.n_cells + H::CPB - 1) / H::CPB;
-        if (grid == 0) return hipSuccess;
-        hipLaunchKernelGGL((dg_operator_gen_kernel<DIM, K, Number, true>), dim3(grid),
-                           dim3(H::BLOCK), 0, s, m, src, e);
+    const int n = m.n_cells;
+    if (n == 0) return hipSuccess;
+    const bool on = gen_kernel_enabled(), node = F::NODE_EXISTS && F::node(n, !e.o2);
+    if constexpr (F::NODE_EXISTS && GenNodeShape<DIM, K>::ENABLED)
+      if (on && node) {
+        hipLaunchKernelGGL((dg_operator_gen_node_kernel<DIM, K, Number>), dim3(n),
+                           dim3(GenNodeShape<DIM, K>::BLOCK), 0, s, m, src, tab, e);
         return hipGetLastError();
       }
-    const int grid = (m.n_cells + G::CPB - 1) / G::CPB;
-    if (grid == 0) return hipSuccess;
-    hipLaunchKernelGGL((dg_operator_gen_kernel<DIM, K, Number>), dim3(grid), dim3(G::BLOCK), 0, s,
-                       m, src, e);
+    if (!on || node) {
+      using S = Shape<DIM, K>;
+      hipLaunchKernelGGL((dg_operator_kernel<DIM, K, Number>), dim3((n + S::CPB - 1) / S::CPB),
+                         dim3(S::BLOCK), 0, s, m, src, tab, e);
+      return hipGetLastError();
+    }
+    if constexpr (GenSmall<DIM, K>::EXISTS)
+      if (GenSmall<DIM, K>::pays(n)) {
+        using H = GenShape<DIM, K, true>;
+        hipLaunchKernelGGL((dg_operator_gen_kernel<DIM, K, Number, true>),
+                           dim3((n + H::CPB - 1) / H::CPB), dim3(H::BLOCK), 0, s, m, src, e);
+        return hipGetLastError();
+      }
+    using G = GenShape<DIM, K>;
+    hipLaunchKernelGGL((dg_operator_gen_kernel<DIM, K, Number>), dim3((n + G::CPB - 1) / G::CPB),
+                       dim3(G::BLOCK), 0, s, m, src, e);
   }
   return hipGetLastError();
 }

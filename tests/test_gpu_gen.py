@@ -2,9 +2,9 @@
 counts that leave the last group part-filled, odd numbers of entries per cell
 (2D, odd N: the flat copies end in a single entry), vectors that are only 8-byte
 aligned, in-place operands, cell scales with inactive cells.  Every output is
-checked against the same sum formed from the kernel's own M^-1 A(src) (which the
-parity tests pin to the oracle): an FMA may round once less, <= 4 ulp of the
-largest term."""
+checked against the same sum formed from the kernel's own M^-1 A(src): an FMA may
+round once less, <= 4 ulp of the largest term; M^-1 A(src) itself, in both
+precisions, against the oracle (the bars of the operator's parity)."""
 import numpy as np
 import pytest
 
@@ -43,6 +43,10 @@ def test_epilogues(dim, nint, k, off):
 
     src, b, c, kk = vec(1), vec(2), vec(3), vec()
     op.apply(src, kk)
+    want, f32 = om.apply(k, src.cpu().numpy()), vec()
+    op.apply(src, f32, precision=X.FP32)
+    for got, tol in ((kk, 1e-12), (f32, 2e-5 * max(1.0, (k / 8) ** 2))):
+        assert np.max(np.abs(got.cpu().numpy() - want)) <= tol * np.max(np.abs(want))
     a1, a2 = 0.37, -1.3
     # the RK stage, o1 over b
     o1, o2 = vec(), vec()
