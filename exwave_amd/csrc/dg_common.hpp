@@ -216,6 +216,8 @@ __device__ __forceinline__ float recip(float x) { return 1.0f / x; }
 // and fused forms against the plain one), so what each of them evaluates in code
 // of its own says which products are fused: explicit FMAs, and no contraction
 // elsewhere (left to itself the compiler fuses a b + c d either way, by context).
+// SAID false (2D k=7, CART_FMAS): its two kernels agree without, and the compiler's own
+// choice schedules better (RK stages 2 to 5 % faster in both precisions).
 __device__ __forceinline__ double fma_of(double a, double b, double c) {
   return __builtin_fma(a, b, c);
 }
@@ -223,11 +225,17 @@ __device__ __forceinline__ float fma_of(float a, float b, float c) {
   return __builtin_fmaf(a, b, c);
 }
 // one row of a face's flux map on (own v_n, own p, neighbour v_n, neighbour p)
-template <typename T>
+template <bool SAID, typename T>
 __device__ __forceinline__ T flux_row(const T *c, T vo, T po, T vn, T pn) {
+  if constexpr (!SAID) return c[0] * vo + c[1] * po + c[2] * vn + c[3] * pn;
   return fma_of(c[3], pn, fma_of(c[2], vn, fma_of(c[1], po, c[0] * vo)));
 }
-// k plus the lifting of the two face values of a line
+// k plus the lifting of one face value, of the two of a line
+template <bool SAID, typename T>
+__device__ __forceinline__ T lift_end(T k, T l, T f) {
+  if constexpr (!SAID) return k + l * f;
+  return fma_of(l, f, k);
+}
 template <typename T>
 __device__ __forceinline__ T lift_ends(T k, T l0, T f0, T l1, T f1) {
   return fma_of(l1, f1, fma_of(l0, f0, k));

@@ -27,10 +27,42 @@
 
 namespace exw {
 
+// The least number of groups of dg_operator_cartp_kernel (below) on a launch with two
+// outputs that runs it (NEVER: none).  Below, its larger groups are spread unevenly over
+// the CUs.  (With one output the staged kernel moves less, and the pair kernel gains nowhere by
+// more than it loses elsewhere.)  RK stage, its time over the staged kernel's at so
+// many groups:
+//   FP64 2D k=2 439 1.04, 793 0.96, 7059 0.89;  k=3 484 1.03, 589 0.98, 1296 0.87;
+//        k=4 281 1.21, 785 1.05, 1452 1.07, 1901 0.97, 44409 0.97;  k=5 281 1.19,
+//        505 0.98, 1210 0.72;  3D k=2 247 to 586 1.00, 980 0.91, 53322 0.97
+//   FP32 2D k=2 652 1.02, 974 0.93;  k=3 265 1.06, 589 0.95;  k=4 1103 0.97, 1452
+//        1.12, 1901 0.93;  k=5 349 1.02, 505 0.96;  k=9 384 1.22, 726 0.86, 2205 1.07,
+//        3314 0.97, 22205 0.95;  k=11 260 0.90, 1378 0.91;  3D k=2 586 1.03, 980 0.93;
+//        k=4 1099 1.11, 6084 1.02, 39754 0.98;  k=5 343 0.98, 1331 0.88
+// Degree 1 gains at every size.  Never (FP32; some sizes gain up to 15 %, others lose
+// up to 37 %): 2D k=7 562 1.12, 25992 1.11;  k=8 265 1.37, 586 0.87, 16418 1.06;
+// k=10 305 1.32, 541 0.83, 15457 1.19;  k=12 273 1.30, 651 0.80, 13807 1.02;  2D k=6;
+// 3D k=3.  FP64 2D k >= 6 and 3D k >= 3 run the pipelined kernel.
+template <int DIM, int K, typename Number>
+constexpr int cart_pairs_from() {
+  constexpr int NEVER = 1 << 30;
+  if constexpr (std::is_same_v<Number, double>) {
+    if (DIM == 3) return K == 1 ? 0 : K == 2 ? 450 : NEVER;
+    return K == 1 ? 0 : K == 2 ? 700 : K == 3 ? 560 : K == 4 ? 1800 : K == 5 ? 500 : NEVER;
+  } else {
+    if (DIM == 3) return K == 1 ? 0 : K == 2 ? 700 : K == 4 ? 10000 : K == 5 ? 500 : NEVER;
+    return K == 1 ? 0 : K == 2 ? 850 : K == 3 ? 560 : K == 4 ? 1800 : K == 5 ? 500
+           : K == 9 ? 2600 : K == 11 ? 256 : NEVER;
+  }
+}
+
+// whether the degree's kernels spell out their FMAs (flux_row)
+template <int DIM, int K>
+constexpr bool CART_FMAS = !(DIM == 2 && K == 7);
+
 #ifndef EXW_CART_GROUP
 #define EXW_CART_GROUP 128
 #endif
-
 
 template <int DIM, int K>
 struct CartShape {
@@ -231,13 +263,13 @@ __device__ __forceinline__ void cart_cell(const DevMesh &mesh, const double *__r
         pn += lo * s_nb[lcB][f][1][n];
       }
       const Number *c = s_fc[lcB][f];
-      const Number fv = flux_row(c, vo, po, vn, pn);
-      const Number fp = flux_row(c + 4, vo, po, vn, pn);
+      const Number fv = flux_row<CART_FMAS<DIM, K>>(c, vo, po, vn, pn);
+      const Number fp = flux_row<CART_FMAS<DIM, K>>(c + 4, vo, po, vn, pn);
 #pragma unroll
       for (int i = 0; i < N; ++i) {
         const Number lw = Number(T.LW[s * N + i]);
-        kv[i] = fma_of(lw, fv, kv[i]);
-        kp[i] = fma_of(lw, fp, kp[i]);
+        kv[i] = lift_end<CART_FMAS<DIM, K>>(kv[i], lw, fv);
+        kp[i] = lift_end<CART_FMAS<DIM, K>>(kp[i], lw, fp);
       }
     }
 #pragma unroll
@@ -311,20 +343,10 @@ __global__ void __launch_bounds__((CartShape<DIM, K>::BLOCK))
 // barriers than dg_operator_cart_kernel (all neighbour fields of the group
 // staged at once where they take up to 24 KB, FULL; else one direction's at a
 // time) and larger groups, so it pays where memory accesses dominate.
-// RK stage, us, dg_operator_cart_kernel -> this one: 2D 301x287 k=5 102 -> 80,
+// cart_pairs_from says which launches run it.  RK stage, us, dg_operator_cart_kernel ->
+// this one: 2D 301x287 k=5 102 -> 80,
 // 512^2 k=3 109 -> 93, 700^2 k=2 192 -> 168, 1000^2 k=1 186 -> 111; 3D 45^3 k=2
-// 109 -> 99, 60^3 k=1 97 -> 62, FP32 40^3 k=4 250 -> 219.
-// Where it was measured faster: sweeps with two outputs and more (with one the
-// staged kernel moves too little to gain, and lost nowhere but at 2D k=5), on at
-// least one group per CU (below, both take their latency, and the staged one's
-// smaller groups spread better: 2D k=4 32^2 6.1 against 7.3 us; degree 1 always
-// gains), for 2D but k=6 (123 against 131 us, FP32), 3D k <= 2, and 3D k=4, 5 with
-// the FP32 operator (FP64 runs the pipelined kernel there; k=3: 116 against 119).
-template <int DIM, int K, typename Number>
-constexpr bool cart_pairs_pay() {
-  return DIM == 2 ? K != 6 : (K <= 2 || (std::is_same_v<Number, float> && (K == 4 || K == 5)));
-}
-
+// 109 -> 99, 60^3 k=1 97 -> 62, FP32 32^3 k=5 204 -> 182.
 template <int DIM, int K, typename Number>
 struct CartLines {
   using G = GenShape<DIM, K>;
@@ -551,8 +573,8 @@ __global__ void __launch_bounds__((CartLines<DIM, K, Number>::BLOCK))
         po += Number(T.L[s * N + i]) * pl[i];
       }
       const Number *c = s_fc[lcB][2 * d + s];
-      fv[s] = flux_row(c, vo, po, tr[s][0], tr[s][1]);
-      fp[s] = flux_row(c + 4, vo, po, tr[s][0], tr[s][1]);
+      fv[s] = flux_row<true>(c, vo, po, tr[s][0], tr[s][1]);
+      fp[s] = flux_row<true>(c + 4, vo, po, tr[s][0], tr[s][1]);
     }
     Number(*ks)[NDP] = s_nb[kp_slot(d)];
 #pragma unroll

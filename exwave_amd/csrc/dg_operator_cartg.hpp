@@ -247,8 +247,8 @@ __global__ void __launch_bounds__((CartGShape<DIM, K>::BLOCK))
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
         const Number *c = s_fc[2 * d + s];
-        fv[s] = flux_row(c, vo[s], po[s], tv[s], tp[s]);
-        fp[s] = flux_row(c + 4, vo[s], po[s], tv[s], tp[s]);
+        fv[s] = flux_row<true>(c, vo[s], po[s], tv[s], tp[s]);
+        fp[s] = flux_row<true>(c + 4, vo[s], po[s], tv[s], tp[s]);
       }
     }
     asm volatile("" ::: "memory");  // reload, do not keep the first loads

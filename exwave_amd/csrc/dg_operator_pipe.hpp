@@ -329,13 +329,13 @@ __device__ __forceinline__ void pipe_line(int line, double *buf, const double *f
       pn += lo * np[n];
     }
     const double *c = fc + 8 * f;
-    const double fv = flux_row(c, vo, po, vn, pn);
-    const double fp = flux_row(c + 4, vo, po, vn, pn);
+    const double fv = flux_row<CART_FMAS<DIM, K>>(c, vo, po, vn, pn);
+    const double fp = flux_row<CART_FMAS<DIM, K>>(c + 4, vo, po, vn, pn);
 #pragma unroll
     for (int i = 0; i < N; ++i) {
       const double lw = T.LW[s * N + i];
-      kv[i] = fma_of(lw, fv, kv[i]);
-      kp[i] = fma_of(lw, fp, kp[i]);
+      kv[i] = lift_end<CART_FMAS<DIM, K>>(kv[i], lw, fv);
+      kp[i] = lift_end<CART_FMAS<DIM, K>>(kp[i], lw, fp);
     }
   });
   double *ov = buf + slot(I0{}, I0{}), *op = buf + slot(I0{}, I1{});

@@ -185,6 +185,22 @@ def test_turnover_pipelined_pools(S, ctx):
         assert _key(mix[q["id"]]) == _key(solo[q["id"]]), q
 
 
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_pair_kernel_pools(S, ctx, prec):
+    """Pools of many small cells (2D k=3: 12288 cells in 64 x 64 solves, k=5: 8192) run
+    dg_operator_cartp_kernel over their cell list, a solve alone the staged kernel:
+    the same bits, with solves that end at different steps."""
+    X, srv = S
+    p = X.FP64 if prec == "fp64" else X.FP32
+    reqs = [dict(id=300 + i, arrival=0.0, dim=2, degree=k, n_refinements=6, rho=1.0 + 0.1 * i,
+                 c=1.2 - 0.1 * i, modes=[1 + i, 2], final_time=t, cfl=0.2)
+            for i, (k, t) in enumerate([(3, 0.008), (3, 0.008), (3, 0.005), (5, 0.004), (5, 0.003)])]
+    mix, _ = srv.run_server(ctx, reqs, lambda _q: p, realtime=False)
+    solo, _ = srv.run_one_at_a_time(ctx, reqs, p)
+    for q in reqs:
+        assert _key(mix[q["id"]]) == _key(solo[q["id"]]), q
+
+
 def test_footprint_matches_pool_size(S, ctx):
     """The size check at submission uses the pool's own per-cell bytes: a
     request whose pool cells (with the pipelined kernel's flux coefficients)
