@@ -443,8 +443,8 @@ __device__ __forceinline__ void column_sum(double *v, int idx, int first, double
 // eigenvectors SV (SV^T W SV = 1), so z = SV3 (1 / sum_e g_e lambda) SV3^T r,
 // the constant left out.  On box cells that is the exact inverse (one
 // iteration); on the deformed membranes 8-14 iterations reach the 1e-13 that
-// plain CG needs 60-150 for.  The relative stop is on r.z, the energy norm of the
-// error in that metric; the absolute one on |r| at the Gauss points.  A cell
+// plain CG needs 60-150 for.  Both stops are on r.z, the energy norm of the error in
+// that metric, relative to the first one.  A cell
 // whose p.Ap is at the bottom of the exponent range (a state that has decayed
 // to 1e-150) ends with what it has: the ratio of two such numbers is noise.
 //
@@ -690,26 +690,17 @@ __global__ void __launch_bounds__((PostColumns<DIM, K>::BLOCK))
     post::column_sum<LPC, BLOCK, 1>(v, idx, lc * LPC, s_red);
     return v[0];
   };
-  // r.z and r.r
-  auto residual = [&](const double *r, const double *z, double (&v)[2]) {
-    v[0] = v[1] = 0.0;
-#pragma unroll
-    for (int j = 0; j < P; ++j) {
-      v[0] += r[j] * z[j];
-      v[1] += r[j] * r[j];
-    }
-    if (!act) v[0] = v[1] = 0.0;
-    post::column_sum<LPC, BLOCK, 2>(v, idx, lc * LPC, s_red);
-  };
-
   double u[P], r[P], p[P];
   div(val, r);  // (val[0..DIM-1] holds the right-hand side's flux)
 #pragma unroll
   for (int j = 0; j < P; ++j) u[j] = 0.0;
   precond(r, p);
   double rz = dot(r, p);
-  const double stop = cfg.rel_tol * cfg.rel_tol * rz, stop_abs = cfg.abs_tol * cfg.abs_tol;
-  const double guard = fmax(1e-5 * stop_abs, 1e4 * 2.2250738585072014e-308);  // as plain CG's
+  // |r| < abs_tol is tested on r.z too, in the first residual's proportion (a sum of
+  // its own costs the iterations 4 %)
+  const double abs2 = cfg.abs_tol * cfg.abs_tol;
+  const double stop = rz * fmax(cfg.rel_tol * cfg.rel_tol, abs2 / dot(r, r));
+  const double guard = fmax(1e-5 * abs2, 1e4 * 2.2250738585072014e-308);  // as plain CG's
   // a zero right-hand side (or NaN) leaves u = 0 (or NaN, through r)
   bool done = !(rz > 0.0);
   if (done && !(rz == 0.0)) u[0] = rz - rz;
@@ -727,12 +718,11 @@ __global__ void __launch_bounds__((PostColumns<DIM, K>::BLOCK))
       }
     }
     precond(r, q);
-    double rn[2];
-    residual(r, q, rn);
+    const double rn = dot(r, q);
     if (!done) {
-      const double beta = rn[0] / rz;
-      rz = rn[0];
-      done = pAp < guard || !(rn[0] > stop) || rn[1] < stop_abs;
+      const double beta = rn / rz;
+      rz = rn;
+      done = pAp < guard || !(rn > stop);
 #pragma unroll
       for (int j = 0; j < P; ++j) p[j] = q[j] + beta * p[j];
     }

@@ -383,12 +383,12 @@ int exw_write_vtu(int dim, int degree, int n_cells, const double *vertices,
  * stops per cell at |r| < EXW_POST_ABS_TOL, |r|/|r0| < EXW_POST_REL_TOL or
  * after EXW_POST_MAX_ITER_FACTOR * (k+2)^dim + 1 iterations (the reference:
  * 1e-20, 1e-11, 6 n, :798-799).  With iterations == NULL the CG is
- * preconditioned and takes a tenth of the iterations: the same cap and absolute
- * tolerance, r being the residual tested with the basis at the Gauss(k+2) points,
- * and the relative tolerance on sqrt(r.z) in place of |r|, z the preconditioned
- * residual (the energy norm of the error).  With counts asked for it is the plain
- * one, whose counts they are.  The two agree to these tolerances, not bit for
- * bit.  Asynchronous on the context's stream. */
+ * preconditioned and takes a tenth of the iterations: the same cap, and both
+ * tolerances on |r0| sqrt(r.z / r0.z0) in place of |r|, z being the preconditioned
+ * residual (r.z is the energy norm of the error) and r the residual in the basis at
+ * the Gauss(k+2) points.  With counts asked for it is the plain one, whose counts
+ * they are.  The two agree to these tolerances, not bit for bit.  Asynchronous on
+ * the context's stream. */
 #define EXW_POST_ABS_TOL 1e-20
 #define EXW_POST_REL_TOL 1e-13
 #define EXW_POST_MAX_ITER_FACTOR 6
