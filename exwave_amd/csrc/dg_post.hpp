@@ -758,6 +758,16 @@ __global__ void __launch_bounds__((PostColumns<DIM, K>::BLOCK))
   }
 }
 
+// Whether p* is summed directly at each point of the error rule instead of by tensor
+// passes: in 2D from k=5 on, where a cell's 7 to 14 lines leave most of a group idle
+// through the passes' barriers, and the direct sums have few terms.  us per call with
+// the readback (about 28), direct / passes: 2D k=4 19881 cells 53.3 / 46.1, k=5 196
+// 29.8 / 32.2, k=7 7744 56.5 / 74.3, k=12 2916 67.7 / 79.2; 3D k=4 2744 141 / 64.
+template <int DIM, int K>
+constexpr bool post_error_direct() {
+  return DIM == 2 && K >= 5;
+}
+
 // ||p* - p_exact||^2 partial sums with QGauss(k+3) (source/explicit_wave.cc:477-484)
 template <int DIM, int K>
 __global__ void __launch_bounds__(256)
@@ -773,6 +783,30 @@ __global__ void __launch_bounds__(256)
   modes_factors<DIM>(modes, t, s_amp);
   const double *xe = tab + T::XE, *we = tab + T::WE;
   double err = 0.0;
+  if constexpr (post_error_direct<DIM, K>()) {
+    for (int i = threadIdx.x; i < E * P; i += 256) s_a[i] = tab[T::IE + i];
+    __syncthreads();
+    const size_t total = (size_t)mesh.n_cells * NE;
+    for (size_t gid = (size_t)blockIdx.x * 256 + threadIdx.x; gid < total;
+         gid += (size_t)gridDim.x * 256) {
+      const int cell = int(gid / NE), q = int(gid % NE);
+      const int qi[2] = {q % E, q / E};
+      double xi[2], x[2], J[4], Ji[4], ex[DIM + 1];
+      xi[0] = xe[qi[0]];
+      xi[1] = xe[qi[1]];
+      const double *V = mesh.vertices + (size_t)cell * NVD, *pc = post + (size_t)cell * NP;
+      multilinear_point<DIM>(V, xi, x);
+      const double jxw = fabs(multilinear_jacobian<DIM>(V, xi, J, Ji)) * we[qi[0]] * we[qi[1]];
+      double val = 0.0;
+      for (int n = 0; n < NP; ++n)
+        val += s_a[qi[0] * P + n % P] * s_a[qi[1] * P + n / P] * pc[n];
+      modes_all<DIM>(modes, s_amp, x, ex);
+      const double d = val - ex[DIM];
+      err += d * d * jxw;
+    }
+    block_partials<1>(&err, red, partial);
+    return;
+  }
   for (int c0 = blockIdx.x * CPB; c0 < mesh.n_cells; c0 += gridDim.x * CPB) {
     const int nc = min(CPB, mesh.n_cells - c0);
     __syncthreads();  // the points of the cells before have been read
