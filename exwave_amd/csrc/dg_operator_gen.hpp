@@ -213,6 +213,29 @@ __device__ __forceinline__ float recip_sqrt(float x) {
   return __builtin_fmaf(0.5f * y, __builtin_fmaf(-x * y, y, 1.0f), y);
 }
 
+// 1/|c| and |c|.  Low-degree 3D cells in FP32 take their length out of the square by a
+// power of two (exact), so that cells of 3e-11 or 3e10 have an area as those of 1 do.
+template <int DIM, int K, typename T>
+__device__ __forceinline__ void norm_of(const T *c, T &inv, T &len) {
+  T n2 = T(0);
+  if constexpr (DIM == 3 && K <= 2 && std::is_same_v<T, float>) {
+    const int e = __builtin_amdgcn_frexp_expf(fmaxf(fmaxf(fabsf(c[0]), fabsf(c[1])), fabsf(c[2])));
+#pragma unroll
+    for (int i = 0; i < DIM; ++i) {
+      const float x = __builtin_amdgcn_ldexpf(c[i], -e);
+      n2 += x * x;
+    }
+    const float y = recip_sqrt(n2);
+    inv = __builtin_amdgcn_ldexpf(y, -e);
+    len = __builtin_amdgcn_ldexpf(n2 * y, e);
+  } else {
+#pragma unroll
+    for (int i = 0; i < DIM; ++i) n2 += c[i] * c[i];
+    inv = recip_sqrt(n2);
+    len = n2 * inv;
+  }
+}
+
 template <int DIM, int K, typename Number, bool SMALL = false>
 __global__ void __launch_bounds__((GenShape<DIM, K, SMALL>::BLOCK))
     __attribute__((amdgpu_waves_per_eu(GenShape<DIM, K, SMALL>::MIN_WAVES)))
@@ -509,13 +532,10 @@ __global__ void __launch_bounds__((GenShape<DIM, K, SMALL>::BLOCK))
     for (int i = 0; i < DIM; ++i) s_jd[lcB][d][i][t] = jd[i];
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-      Number na2 = Number(0), det = Number(0);
+      Number det = Number(0), inv, na;
 #pragma unroll
-      for (int i = 0; i < DIM; ++i) {
-        na2 += av[s][i] * av[s][i];
-        det += av[s][i] * jd[i];
-      }
-      const Number inv = recip_sqrt(na2), na = na2 * inv;
+      for (int i = 0; i < DIM; ++i) det += av[s][i] * jd[i];
+      norm_of<DIM, K>(av[s], inv, na);
       const Number sg = (s != 0) == (det > Number(0)) ? Number(1) : Number(-1);
       Number vp = Number(0), vm = Number(0);
 #pragma unroll

@@ -71,3 +71,23 @@ def test_epilogues(dim, nint, k, off):
     near(o1[on], (b + a1 * sc * kk)[on], b, 2 * kk)
     near(o2[on], (b + a1 * sc * kk + a2 * sc * kk)[on], b, 4 * kk)
     assert torch.equal(o1[~on], w1[~on]) and torch.equal(o2[~on], w2[~on])
+
+
+@pytest.mark.parametrize("dim,nint,k", [(2, 5, 1), (2, 5, 3), (3, 3, 1), (3, 3, 2)])
+@pytest.mark.parametrize("size", [1e-10, 1.0, 1e11])
+def test_fp32_range_of_lengths(dim, nint, k, size):
+    """The FP32 operator on meshes of any unit of length: the squares of a face's area
+    (1e-42, 1e42 here in 3D) are outside the range of 32 bits, areas and volumes are
+    not.  The bar of the FP32 parity tests."""
+    import torch
+
+    import exwave_amd as X
+    print("gen lengths", dim, nint, k, size, flush=True)
+    om = O.Mesh(dim, nint, 0, O.TRANSFORM_REFERENCE_SINE, 0.1, 3)
+    V = np.ctypeslib.as_array(om._m.contents.vertices, shape=(om.n_cells, 1 << dim, dim))
+    V *= size
+    op = X.WaveOperator(X.Context(0), dim, k, om.vertices, om.neighbor, om.rho, om.speed)
+    u = np.random.default_rng(3).standard_normal(op.n_dofs)
+    want, got = om.apply(k, u), op.new_vector()
+    op.apply(torch.from_numpy(u).cuda(), got, precision=X.FP32)
+    assert np.max(np.abs(got.cpu().numpy() - want)) <= 2e-5 * np.max(np.abs(want))
