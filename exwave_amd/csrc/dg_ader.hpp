@@ -555,7 +555,8 @@ __global__ void __launch_bounds__((CkGroup<DIM, K>::BLOCK))
 //        22.9 / 20.6;  k=7 512 15.5 / 17.1, 1000 26.8 / 20.1
 // Never: 3D k=5 (lines fill 36 of a wave's 64 lanes: 4913 cells 38.9 / 41.8), k=8, 9
 // (two waves per direction, registers: 592 / 632 at k=9, 5832 cells), 2D k=12, and
-// FP32 k=3 (2D 83521 cells 13.0 / 14.1, 3D 15625 13.0 / 15.1).
+// FP32 2D k=3 (83521 cells 13.0 / 14.1).  FP32 3D k=3 loses to 30000 cells (15625 13.0 /
+// 15.1) and gains with the fused kernel from 10^5 on (262144: 501 / 492 per step).
 template <int DIM, int K, typename Number>
 struct CkLinesFrom {
   static constexpr int NEVER = 1 << 30;
@@ -567,7 +568,7 @@ struct CkLinesFrom {
              : K == 11 ? 3584 : NEVER;
     } else {
       if (D) return K <= 2 ? 0 : K == 3 ? 128 : K == 4 ? 512 : K == 6 || K == 7 ? 384 : NEVER;
-      return K <= 2 ? 0 : K == 4 ? 1792 : K == 6 ? 1280 : K == 7 ? 768 : NEVER;
+      return K <= 2 ? 0 : K == 3 ? 50000 : K == 4 ? 1792 : K == 6 ? 1280 : K == 7 ? 768 : NEVER;
     }
   }
   static constexpr bool ALWAYS = groups() == 0, EXISTS = groups() < NEVER;
