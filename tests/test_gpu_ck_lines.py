@@ -1,5 +1,5 @@
-"""The Cauchy-Kowalevski integral on box cells (ader_ck_lines_kernel: one lane per
-line, whole waves per direction) against the oracle: cells with a different size in
+"""The Cauchy-Kowalevski integral on box cells (ader_ck_lines_kernel, one lane per
+line, or ader_ck_kernel, one lane per node) against the oracle: cells with a different size in
 each direction, varying media, groups that hold several cells with the last one
 part-filled, odd numbers of entries per cell, vectors that start on an odd 8 bytes,
 with and without the given first derivative, on an interval away from its
@@ -14,7 +14,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("dim,k,nint", [
     (2, 1, 5), (2, 2, 5), (2, 3, 3), (2, 4, 5), (2, 5, 3), (2, 7, 3), (2, 9, 3), (2, 11, 2),
-    (2, 12, 3), (3, 1, 3), (3, 2, 3), (3, 3, 3), (3, 4, 2), (3, 5, 2), (3, 6, 2), (3, 9, 2)])
+    (2, 12, 3), (3, 1, 3), (3, 2, 3), (3, 3, 3), (3, 4, 2), (3, 5, 2), (3, 6, 2), (3, 9, 2),
+    (2, 6, 3), (2, 8, 3), (2, 10, 2), (3, 7, 2), (3, 8, 2)])
 def test_ck_lines_vs_oracle(dim, k, nint):
     import torch
 

@@ -1,7 +1,7 @@
 """The output tick's kernels at the edges of their layouts: the preconditioned
 solver of exw_post_pressure (a call without iteration counts) against the
-oracle's CG and against the plain CG kernel (a call with them), and the
-factored L2 errors against the oracle's direct sums.
+oracle's CG and against the plain CG kernel (a call with them), the factored L2
+errors and the error of p*, the energy and the projection against the oracle.
 
 Columns per cell of the solver: 3..14 (2D, several cells per wave, cell counts
 that leave the last group part-filled), 9..100 in 3D (49 and 64 in one wave, 81
@@ -88,6 +88,30 @@ def test_post_pcg_scales(X, dim, nint, k):
         assert float(post.abs().max()) <= 4 * top * s, e
         if e == 3:
             assert float((post - s * one).abs().max()) <= 1e-10 * top * s
+
+
+@pytest.mark.parametrize("case", POST + [(2, 7, O.TRANSFORM_REFERENCE_SINE, 0.1, 5),
+                                         (2, 6, O.TRANSFORM_AXIS_2PI, 0.04, 9)],
+                         ids=lambda c: "d%d_n%d_t%d_k%d" % (c[0], c[1], c[2], c[4]))
+def test_tick_norms(X, case):
+    """The error of p* (tensor passes; direct sums in 2D from degree 5 on), the energy
+    and the projection against the oracle: sums of at most 10^5 terms of one sign in
+    another order, 1e-12; single evaluations of the modes, 1e-14."""
+    import torch
+    dim, nint, tr, fac, k = case
+    print("tick norms", case, flush=True)
+    om, op, u = _setup(X, *case)
+    mm = [[1] * dim, [2] + [1] * (dim - 1)]
+    e, m = O.Exact.make(dim, mm, [1.0, 0.3]), X.Modes.make(dim, mm, [1.0, 0.3])
+    want = om.project(k, e, 0.3)
+    got = op.new_vector()
+    op.project(m, 0.3, got)
+    assert np.max(np.abs(got.cpu().numpy() - want)) <= 1e-14 * np.max(np.abs(want))
+    en = om.energy(k, u)
+    assert abs(op.energy(torch.from_numpy(u).cuda()) - en) <= 1e-12 * en
+    post = np.random.default_rng(k).standard_normal(op.n_post)
+    err = om.post_error(k, e, 0.3, post)
+    assert abs(op.post_error(m, 0.3, torch.from_numpy(post).cuda()) - err) <= 1e-12 * err
 
 
 @pytest.mark.parametrize("dim,nint,k", [(2, 5, 1), (2, 3, 6), (2, 2, 12), (3, 3, 1), (3, 3, 4),
