@@ -156,8 +156,8 @@ __global__ void __launch_bounds__((AderFusedShape<DIM, K>::BLOCK))
 // the neighbour traces of faces 2d, 2d+1 at its face
 // points straight from the neighbours' nodes in memory, instead of the
 // neighbours' fields being staged in LDS.  The LDS of the sweep shrinks to the
-// cell's fields and the lines' dp/dt shares (3D k=4: 7.4 KB; the union is then
-// the CK's 7 KB instead of 16 KB): 3D k=4 64^3 90.1 -> 97.9, k=5 40^3 71.8 -> 84.0,
+// cell's fields and the lines' dp/dt shares (3D k=4: 7.4 KB, which the CK's 7 KB fit
+// into, instead of 16 KB): 3D k=4 64^3 90.1 -> 97.9, k=5 40^3 71.8 -> 84.0,
 // k=3 64^3 115 -> 127 GDoF/s per ADER step (FP64, with the CK of one lane per node).
 // With the CK in line form (ader_ck_lines_kernel's), on another card: k=4 94.0 ->
 // 102.3, k=3 126.7 -> 131.2, FP32 k=4 113.4 -> 118.4, k=3 138.4 -> 140.4 GDoF/s; the sweep half's memory

@@ -84,7 +84,8 @@ struct GenShape {
   static constexpr int PPC = (NF * ND + 1) / 2, NPP = (CPB * PPC + BLOCK - 1) / BLOCK;
   static constexpr bool PREFETCH_ALL = NPP <= 2;
   // waves per SIMD to hold the registers to, one or two below the compiler's
-  // own choice (no spills)
+  // own choice (no vector register spills; the matrices' constants spill scalar
+  // registers to vector lanes, 8 to 30 at k=5, 100 to 800 from 2D k=8 and 3D k=8 on)
   static constexpr int MIN_WAVES = DIM == 3 ? (K <= 5 ? 5 : 4) : (K <= 3 ? 6 : 4);
 };
 
@@ -110,8 +111,9 @@ struct GenSmall {
 // both, and at 2D k >= 9 the code leaves the instruction cache.  The node forms read
 // their tables from LDS in short loops.  us per RK stage (two outputs) and, behind
 // the bar, per single-output sweep, node form / line form:
-//   FP64 2D k=1 332929 cells 60 / 50 | 41 / 43;  k=3 11449 8.1 / 8.0 | 5 % lost;  k=4
-//        676 6.1 / 5.5, 1600 6.0 / 6.4, 3969 6.9 / 7.8, 7396 10.9 / 9.4;  k=5 2809 8.8
+//   FP64 2D k=1 58212 cells 10.5 / 11.3 (just before the node form's 64-cell groups need a
+//        second round of the CUs), 332929 60 / 50 | 41 / 43;  k=3 11449 8.1 / 8.0 | 5 %
+//        lost;  k=4 676 6.1 / 5.5, 1600 6.0 / 6.4, 3969 6.9 / 7.8, 7396 10.9 / 9.4;  k=5 2809 8.8
 //        / 8.7 | 21 % lost, 9216 15.8 / 12.1;  k=6 2025 7.4 / 8.8, 6724 13.5 / 12.4;
 //        k=7 2916 9.2 / 9.6, 5184 12.9 / 11.0;  k=8 2304 10.9 / 11.7, 4096 15.7 /
 //        13.5;  k=9 1849 9.7 / 12.0, 3364 14.6 / 13.6;  k=10 841 7.9 / 12.4, 5476 24.7
@@ -137,7 +139,7 @@ struct GenForms {
   static constexpr bool D = std::is_same_v<Number, double>;
   static constexpr int from(bool single) {
     if constexpr (DIM == 2) {
-      if (K == 1) return D && single ? 30000 : NEVER;
+      if (K == 1) return D ? (single ? 30000 : 50000) : NEVER;
       if (K == 3) return single ? 6000 : NEVER;
       if (K == 4) return 1200;
       if (K == 5) return D && !single ? NEVER : 600;
@@ -146,22 +148,20 @@ struct GenForms {
     return K >= 5 ? 0 : NEVER;
   }
   static constexpr int to(bool single) {
-    constexpr int f64_2d[13] = {0,    0,    0,    0,    6000,  0,    5500,
-                                4096, 3000, 3000, 12000, 9000, 9000},
-                  f64_2d_single[13] = {0,    NEVER, 0,   32000, 6000,  7500,  5500,
-                                       4096, 3000, 3000, NEVER, 16384, NEVER},
-                  f32_2d[13] = {0,    0,    0,     0,     11000, 7500, 4096,
-                                3584, 8192, 16384, 32768, 12000, NEVER},
-                  f32_2d_single[13] = {0,    0,     0,     0,     11000, 7500, 4096,
-                                       3584, 24000, NEVER, NEVER, NEVER, NEVER},
-                  f64_3d[10] = {0, 0, 0, 0, 0, 2500, 512, 448, 1800, NEVER},
-                  f64_3d_single[10] = {0, 0, 0, 0, 0, NEVER, 512, 448, 2800, NEVER},
-                  f32_3d[10] = {0, 0, 0, 0, 0, 800, 512, 3500, 1152, 448},
-                  f32_3d_single[10] = {0, 0, 0, 0, 0, 2000, 512, 6000, 1152, 448};
-    if constexpr (DIM == 2)
-      return (D ? (single ? f64_2d_single : f64_2d) : (single ? f32_2d_single : f32_2d))[K];
-    else
-      return (D ? (single ? f64_3d_single : f64_3d) : (single ? f32_3d_single : f32_3d))[K];
+    constexpr int N = NEVER;
+    // [FP64 two outputs, FP64 single, FP32 two outputs, FP32 single][degree]
+    constexpr int to_2d[4][13] = {
+        {0, 65536, 0, 0, 6000, 0, 5500, 4096, 3000, 3000, 12000, 9000, 9000},
+        {0, N, 0, 32000, 6000, 11000, 5500, 7000, 3000, 3000, N, 16384, N},
+        {0, 0, 0, 0, 11000, 7500, 4096, 3584, 8192, 16384, 32768, 12000, N},
+        {0, 0, 0, 17000, 11000, 7500, 4096, 3584, 24000, N, N, N, N}};
+    constexpr int to_3d[4][10] = {{0, 0, 0, 0, 0, 2500, 576, 448, 1800, N},
+                                  {0, 0, 0, 0, 0, N, 576, 448, 2800, N},
+                                  {0, 0, 0, 0, 0, 800, 576, 3500, 1152, 448},
+                                  {0, 0, 0, 0, 0, 2000, 576, 6000, 1152, 448}};
+    const int row = (D ? 0 : 2) + (single ? 1 : 0);
+    if constexpr (DIM == 2) return to_2d[row][K];
+    else return to_3d[row][K];
   }
   // (the node form's offsets into the vectors have 32 bits)
   static bool node(int n, bool single) {

@@ -367,7 +367,9 @@ struct PostColumns {
   static constexpr int NPL = DIM == 2 ? P * PP : P * P * PP;  // LDS entries of a tensor
   static constexpr int CPB = LPC <= 64 ? 64 / LPC : 1;
   static constexpr int BLOCK = LPC <= 64 ? 64 : (LPC + 63) / 64 * 64;
-  // columns of up to 6 points (3D) or 9 (2D) fit 256 registers: two waves per SIMD
+  // columns of up to 6 points (3D) or 9 (2D) are held to 256 registers, two waves per
+  // SIMD (the two largest spill 11 and 4 vector registers; the matrices' scalar
+  // registers spill to vector lanes from 2D k=3 and 3D k=2 on)
   static constexpr int MIN_WAVES = P <= (DIM == 2 ? 9 : 6) ? 2 : 1;
 };
 

@@ -10,17 +10,19 @@ import oracle as O
 
 pytestmark = pytest.mark.gpu
 
-CASES = [(2, 1, 0, 173), (2, 1, 0, 174), (2, 3, 0, 77), (2, 3, 1, 78), (2, 3, 1, 123), (2, 3, 0, 95), (2, 3, 0, 179), (2, 4, 0, 34), (2, 4, 0, 35), (2, 4, 0, 77), (2, 4, 0, 79),
-         (2, 5, 0, 24), (2, 5, 0, 25), (2, 5, 0, 86), (2, 5, 0, 87), (2, 6, 0, 74), (2, 6, 0, 76),
-         (2, 7, 0, 63), (2, 7, 0, 65), (2, 8, 0, 54), (2, 8, 0, 57), (2, 9, 0, 54), (2, 9, 0, 55),
-         (2, 10, 0, 109), (2, 10, 0, 111), (2, 11, 0, 94), (2, 11, 0, 96), (2, 12, 0, 96),
-         (3, 5, 0, 13), (3, 5, 0, 14), (3, 6, 0, 7), (3, 6, 0, 8), (3, 7, 0, 7), (3, 7, 0, 8),
-         (3, 8, 0, 12), (3, 8, 0, 13), (3, 9, 0, 3),
-         (2, 4, 1, 104), (2, 4, 1, 106), (2, 5, 1, 86), (2, 5, 1, 88), (2, 6, 1, 63), (2, 6, 1, 65),
-         (2, 7, 1, 59), (2, 7, 1, 61), (2, 8, 1, 90), (2, 8, 1, 92), (2, 9, 1, 127), (2, 9, 1, 129),
-         (2, 11, 1, 109), (2, 11, 1, 111), (2, 12, 1, 30), (3, 5, 1, 9), (3, 5, 1, 10), (3, 5, 1, 13),
-         (3, 6, 1, 8), (3, 7, 1, 15), (3, 7, 1, 16), (3, 8, 1, 10), (3, 8, 1, 11), (3, 9, 1, 7),
-         (3, 9, 1, 8)]
+CASES = [(2, 1, 0, 173), (2, 1, 0, 174), (2, 1, 0, 224), (2, 1, 0, 257), (2, 3, 0, 77),
+         (2, 3, 0, 95), (2, 3, 0, 179), (2, 4, 0, 34), (2, 4, 0, 35), (2, 4, 0, 77),
+         (2, 4, 0, 79), (2, 5, 0, 24), (2, 5, 0, 25), (2, 5, 0, 86), (2, 5, 0, 87),
+         (2, 5, 0, 104), (2, 5, 0, 106), (2, 6, 0, 74), (2, 6, 0, 76), (2, 7, 0, 63),
+         (2, 7, 0, 65), (2, 7, 0, 85), (2, 8, 0, 54), (2, 8, 0, 57), (2, 9, 0, 54),
+         (2, 9, 0, 55), (2, 10, 0, 109), (2, 10, 0, 111), (2, 11, 0, 94), (2, 11, 0, 96),
+         (2, 12, 0, 96), (3, 5, 0, 13), (3, 5, 0, 14), (3, 6, 0, 8), (3, 6, 0, 9), (3, 7, 0, 7),
+         (3, 7, 0, 8), (3, 8, 0, 12), (3, 8, 0, 13), (3, 9, 0, 3), (2, 3, 1, 78), (2, 3, 1, 123),
+         (2, 3, 1, 131), (2, 4, 1, 104), (2, 4, 1, 106), (2, 5, 1, 86), (2, 5, 1, 88),
+         (2, 6, 1, 63), (2, 6, 1, 65), (2, 7, 1, 59), (2, 7, 1, 61), (2, 8, 1, 90),
+         (2, 8, 1, 92), (2, 9, 1, 127), (2, 9, 1, 129), (2, 11, 1, 109), (2, 11, 1, 111),
+         (2, 12, 1, 30), (3, 5, 1, 9), (3, 5, 1, 10), (3, 5, 1, 13), (3, 6, 1, 8), (3, 6, 1, 9),
+         (3, 7, 1, 15), (3, 7, 1, 16), (3, 8, 1, 10), (3, 8, 1, 11), (3, 9, 1, 7), (3, 9, 1, 8)]
 
 
 @pytest.mark.parametrize("dim,k,fp32,nint", CASES)
