@@ -356,7 +356,7 @@ __global__ void __launch_bounds__((AderFusedGShape<DIM, K>::BLOCK), (AderFusedGS
         Number dv = Number(0);
 #pragma unroll
         for (int m = 0; m < N; ++m) dv += Number(T.DT[i * N + m]) * vl[m];
-        const Number k = lift_ends(cvp * dv, Number(T.LW[i]), fp[0], Number(T.LW[N + i]), fp[1]);
+        const Number k = lift_ends<true>(cvp * dv, Number(T.LW[i]), fp[0], Number(T.LW[N + i]), fp[1]);
         s_kp[d][base + i * sd] = k;
       }
     }
@@ -370,7 +370,7 @@ __global__ void __launch_bounds__((AderFusedGShape<DIM, K>::BLOCK), (AderFusedGS
         Number gp = Number(0);
 #pragma unroll
         for (int m = 0; m < N; ++m) gp += Number(T.D[i * N + m]) * pl[m];
-        const Number k = lift_ends(cvv * gp, Number(T.LW[i]), fv[0], Number(T.LW[N + i]), fv[1]);
+        const Number k = lift_ends<true>(cvv * gp, Number(T.LW[i]), fv[0], Number(T.LW[N + i]), fv[1]);
         s_u[d][base + i * sd] = k;
       }
     }

@@ -216,8 +216,9 @@ __device__ __forceinline__ float recip(float x) { return 1.0f / x; }
 // and fused forms against the plain one), so what each of them evaluates in code
 // of its own says which products are fused: explicit FMAs, and no contraction
 // elsewhere (left to itself the compiler fuses a b + c d either way, by context).
-// SAID false (2D k=7, CART_FMAS): its two kernels agree without, and the compiler's own
-// choice schedules better (RK stages 2 to 5 % faster in both precisions).
+// SAID false (CART_FMAS: 2D k=7, 3D k >= 8): the degree's two kernels agree without, and
+// the compiler's own choice schedules better (RK stages at 2D k=7 2 to 5 %, at 3D k=8 and
+// 9 1 to 2 %; at 3D k=7 it loses 2 % of the single-output sweeps).
 __device__ __forceinline__ double fma_of(double a, double b, double c) {
   return __builtin_fma(a, b, c);
 }
@@ -236,9 +237,9 @@ __device__ __forceinline__ T lift_end(T k, T l, T f) {
   if constexpr (!SAID) return k + l * f;
   return fma_of(l, f, k);
 }
-template <typename T>
+template <bool SAID, typename T>
 __device__ __forceinline__ T lift_ends(T k, T l0, T f0, T l1, T f1) {
-  return fma_of(l1, f1, fma_of(l0, f0, k));
+  return lift_end<SAID>(lift_end<SAID>(k, l0, f0), l1, f1);
 }
 
 template <typename T>

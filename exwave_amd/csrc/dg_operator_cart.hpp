@@ -58,7 +58,7 @@ constexpr int cart_pairs_from() {
 
 // whether the degree's kernels spell out their FMAs (flux_row)
 template <int DIM, int K>
-constexpr bool CART_FMAS = !(DIM == 2 && K == 7);
+constexpr bool CART_FMAS = !(DIM == 2 ? K == 7 : K >= 8);
 
 #ifndef EXW_CART_GROUP
 #define EXW_CART_GROUP 128
@@ -582,7 +582,7 @@ __global__ void __launch_bounds__((CartLines<DIM, K, Number>::BLOCK))
       Number dv = Number(0);
 #pragma unroll
       for (int m = 0; m < N; ++m) dv += Number(T.DT[i * N + m]) * vl[m];
-      const Number k = lift_ends(cvp * dv, Number(T.LW[i]), fp[0], Number(T.LW[N + i]), fp[1]);
+      const Number k = lift_ends<true>(cvp * dv, Number(T.LW[i]), fp[0], Number(T.LW[N + i]), fp[1]);
       ks[lcB][base + i * sd] = k;
     }
 #pragma unroll
@@ -590,7 +590,7 @@ __global__ void __launch_bounds__((CartLines<DIM, K, Number>::BLOCK))
       Number gp = Number(0);
 #pragma unroll
       for (int m = 0; m < N; ++m) gp += Number(T.D[i * N + m]) * pl[m];
-      const Number k = lift_ends(cvv * gp, Number(T.LW[i]), fv[0], Number(T.LW[N + i]), fv[1]);
+      const Number k = lift_ends<true>(cvv * gp, Number(T.LW[i]), fv[0], Number(T.LW[N + i]), fv[1]);
       s_u[lcB][d][base + i * sd] = k;  // (over v_d, which only this lane reads)
     }
   });

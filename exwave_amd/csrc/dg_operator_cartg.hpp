@@ -247,8 +247,8 @@ __global__ void __launch_bounds__((CartGShape<DIM, K>::BLOCK))
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
         const Number *c = s_fc[2 * d + s];
-        fv[s] = flux_row<true>(c, vo[s], po[s], tv[s], tp[s]);
-        fp[s] = flux_row<true>(c + 4, vo[s], po[s], tv[s], tp[s]);
+        fv[s] = flux_row<CART_FMAS<DIM, K>>(c, vo[s], po[s], tv[s], tp[s]);
+        fp[s] = flux_row<CART_FMAS<DIM, K>>(c + 4, vo[s], po[s], tv[s], tp[s]);
       }
     }
     asm volatile("" ::: "memory");  // reload, do not keep the first loads
@@ -261,7 +261,8 @@ __global__ void __launch_bounds__((CartGShape<DIM, K>::BLOCK))
         Number dv = Number(0);
 #pragma unroll
         for (int m = 0; m < N; ++m) dv += Number(T.DT[i * N + m]) * vl[m];
-        const Number k = lift_ends(cvp * dv, Number(T.LW[i]), fp[0], Number(T.LW[N + i]), fp[1]);
+        const Number k = lift_ends<CART_FMAS<DIM, K>>(cvp * dv, Number(T.LW[i]), fp[0],
+                                                      Number(T.LW[N + i]), fp[1]);
         s_kp[d][base + i * sd] = k;
       }
     }
@@ -275,7 +276,8 @@ __global__ void __launch_bounds__((CartGShape<DIM, K>::BLOCK))
         Number gp = Number(0);
 #pragma unroll
         for (int m = 0; m < N; ++m) gp += Number(T.D[i * N + m]) * pl[m];
-        const Number k = lift_ends(cvv * gp, Number(T.LW[i]), fv[0], Number(T.LW[N + i]), fv[1]);
+        const Number k = lift_ends<CART_FMAS<DIM, K>>(cvv * gp, Number(T.LW[i]), fv[0],
+                                                      Number(T.LW[N + i]), fv[1]);
         s_u[d][base + i * sd] = k;
       }
     }
