@@ -161,7 +161,7 @@ __global__ void __launch_bounds__((AderFusedShape<DIM, K>::BLOCK))
 // k=3 64^3 115 -> 127 GDoF/s per ADER step (FP64, with the CK of one lane per node).
 // With the CK in line form (ader_ck_lines_kernel's), on another card: k=4 94.0 ->
 // 102.3, k=3 126.7 -> 131.2, FP32 k=4 113.4 -> 118.4, k=3 138.4 -> 140.4 GDoF/s; the sweep half's memory
-// latency and the VALU (5.3e8 instructions at k=4) share the time at 12 groups per
+// latency and the VALU (5.4e8 instructions at k=4) share the time at 12 groups per
 // CU.  The FP32 operator keeps the staged form.
 // The arithmetic is dg_operator_cart_kernel's expression for expression (the
 // traces' chains over the same values, the line phase in the three passes of
