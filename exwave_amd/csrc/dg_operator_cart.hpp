@@ -56,6 +56,18 @@ constexpr int cart_pairs_from() {
   }
 }
 
+// Whether a launch of so many groups runs it: not just beyond one full round of them
+// over the CUs (5, 6 or 7 a CU), where the last, nearly empty round costs more than the
+// pairs gain (3D k=2 FP64 1449 groups 1.08, FP32 1591 1.10; 2D k=3 FP32 1893 1.05).
+template <int DIM, int K, typename Number>
+constexpr bool cart_pairs_pay(int groups) {
+  constexpr bool D = std::is_same_v<Number, double>;
+  constexpr int round =
+      DIM == 3 && K == 2 ? (D ? 1280 : 1536) : DIM == 2 && K == 3 && !D ? 1792 : 0;
+  return groups >= cart_pairs_from<DIM, K, Number>() &&
+         !(round && groups > round && groups <= round + round / 6);
+}
+
 // whether the degree's kernels spell out their FMAs (flux_row)
 template <int DIM, int K>
 constexpr bool CART_FMAS = !(DIM == 2 ? K == 7 : K >= 8);

@@ -173,11 +173,10 @@ hipError_t launch_op(const DevMesh &m, const double *src, const double *tab,
     // box cells: node/line/node kernel with compile-time 1D matrices
     using CS = CartShape<DIM, K>;
     const int n = e.cell_list ? e.n_list : m.n_cells;
-    constexpr int pairs_from = cart_pairs_from<DIM, K, Number>();
-    if constexpr (pairs_from < (1 << 30)) {
+    if constexpr (cart_pairs_from<DIM, K, Number>() < (1 << 30)) {
       using G = GenShape<DIM, K>;
       const int groups = (n + G::CPB - 1) / G::CPB;
-      if (e.o2 && groups > 0 && groups >= pairs_from) {
+      if (e.o2 && groups > 0 && cart_pairs_pay<DIM, K, Number>(groups)) {
         hipLaunchKernelGGL((dg_operator_cartp_kernel<DIM, K, Number>), dim3(groups),
                            dim3(G::BLOCK), 0, s, m, src, e);
         return hipGetLastError();

@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 CASES = [(2, 1, 9), (2, 2, 74), (2, 3, 65), (2, 4, 56), (2, 5, 51), (2, 9, 40), (2, 12, 33),
          (3, 1, 5), (3, 2, 13)]
 # the smallest launches of the degrees whose line lies higher than these
-CASES += [(2, 2, 135), (2, 3, 95), (2, 4, 147), (2, 5, 71), (3, 2, 17)]
+CASES += [(2, 2, 135), (2, 3, 95), (2, 4, 147), (2, 5, 71), (3, 2, 17), (3, 2, 23)]
 FP32_ONLY = [(2, 9, 125), (2, 11, 36), (3, 4, 28), (3, 5, 8), (2, 7, 46), (2, 8, 43), (3, 4, 9), (3, 5, 7)]
 
 
