@@ -95,7 +95,12 @@ struct GenShape {
 // small launches run this kernel (GenForms).  2D, ten launches in us, small against
 // full groups: k=4 506 cells (43 full groups) 54.0 against 64.8, k=5 361 cells (37)
 // 56 against 71; near 230 full groups the small ones take 77 and 82, the full ones
-// 68 and 76: the lines cross between 100 and 160 full groups.
+// 68 and 76: the lines cross between 100 and 160 full groups.  3D, us per RK stage,
+// full / small, FP64 and FP32: k=2 125 cells (18 groups) 6.3 / 5.8, 6.1 / 5.7, 729 (104)
+// 6.4 / 6.3, 6.2 / 6.0, 1331 (190) 6.6 / 7.3, 6.4 / 6.6; k=3 125 (31) 7.0 / 6.2, 6.7 /
+// 5.9, 512 (128) 7.3 / 6.7, 6.9 / 6.1, 1000 (250) 7.7 / 8.5, 7.4 / 7.5; k=4 216 (108)
+// 7.4 / 7.0, 7.1 / 6.8, 343 (172) 7.8 / 8.1, 7.4 / 7.4.  2D FP32 k=4 400 cells (33) 6.4 /
+// 5.6, k=5 361 (37) 7.0 / 5.8.  2D k=3: within 4 % of each other below the line.
 template <int DIM, int K>
 struct GenSmall {
   static constexpr bool EXISTS = (DIM == 2 ? K >= 3 && K <= 5 : K >= 2) &&
