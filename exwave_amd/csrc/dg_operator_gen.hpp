@@ -110,12 +110,16 @@ struct GenSmall {
 
 // Which launches over general cells run the kernels with one lane per node
 // (dg_operator_gen_node_kernel, below 48 nodes dg_operator_kernel) instead of this
-// file's line form: those over from <= n < to cells; `single`: the launch has one
-// output.  The line form's matrices are constants of its unrolled code, which every
+// file's line form: those over from <= n < to cells; `single`: the launch only writes
+// the operator's result.  One output that accumulates (the last stage of a time step,
+// the sweep of an ADER step) goes by the two-output line: it costs the line form no more
+// than its neighbours in the step, and the node form 3 to 15 % (ADER step, us, node /
+// line form: FP64 2D k=1 332929 cells 67.6 / 62.7, k=3 18769 22.8 / 20.4, k=5 8281 35.9 /
+// 31.2).  The line form's matrices are constants of its unrolled code, which every
 // launch fetches once, and its chain of barriers is longer: small launches wait for
 // both, and at 2D k >= 9 the code leaves the instruction cache.  The node forms read
 // their tables from LDS in short loops.  us per RK stage (two outputs) and, behind
-// the bar, per single-output sweep, node form / line form:
+// the bar, per plain sweep, node form / line form:
 //   FP64 2D k=1 58212 cells 10.5 / 11.3 (just before the node form's 64-cell groups need a
 //        second round of the CUs), 332929 60 / 50 | 41 / 43;  k=3 11449 8.1 / 8.0 | 5 %
 //        lost;  k=4 676 6.1 / 5.5, 1600 6.0 / 6.4, 3969 6.9 / 7.8, 7396 10.9 / 9.4;  k=5 2809 8.8
@@ -138,13 +142,23 @@ struct GenSmall {
 //     3D k=5 729 9.8 / 9.9, 1000 12.1 / 11.2 | 13 % lost, 2197 23.6 / 21.6;  k=6 343
 //       9.6 / 10.3, 729 16.4 / 12.7;  k=7 1728 39 / 41, 4096 86 / 82;  k=8 729 28.7 /
 //       29.7, 1331 50.8 / 49.6;  k=9 216 16.2 / 18.5, 512 29.3 / 27.4
+// From a sweep in steps of 12 % of the cells, line form's time over the node form's just
+// below and above the line: FP64 2D k=4 5112 cells 1.15, 5700 0.78 (one round
+// of the node form's groups ends between), k=7 3248 1.02, 4095 0.96, k=8 2304 1.07, 2915
+// 0.97, k=9 2304 1.05, 2915 0.95, 3D k=7 252 1.22, 288 0.96, k=8 1573 1.02, 1728 0.97; FP32 2D k=8 9024 1.01, 10100 0.93,
+// k=9 14160 1.02, 15875 0.92, k=11 9024 1.05, 10100 0.96, 3D k=8 810 1.04, 1000 0.96, k=9 252
+// 1.16, 441 0.95.  FP32 2D k=8 and 9 just below one full round of the line form's groups: 5700
+// 1.02, 6399 0.93, 7140 0.86, 8010 1.00; 5112 1.05, 5700 0.95, 6399 1.21.  Plain sweeps: FP64 2D
+// k=1 22201 0.96, 27889 1.04, k=3 15875 1.09, 17689 0.93, k=5 5112 1.07, 5700 0.85, k=7 3660
+// 1.00, 5112 0.92, k=11 11236 1.00, 14160 0.99; FP32 k=3 15875 1.08, 17689 0.89, k=5 5112 1.07,
+// 5700 0.86, k=8 12656 1.04, 14160 0.97.
 template <int DIM, int K, typename Number>
 struct GenForms {
   static constexpr int NEVER = 1 << 30;
   static constexpr bool D = std::is_same_v<Number, double>;
   static constexpr int from(bool single) {
     if constexpr (DIM == 2) {
-      if (K == 1) return D ? (single ? 30000 : 50000) : NEVER;
+      if (K == 1) return D ? (single ? 24000 : 50000) : NEVER;
       if (K == 3) return single ? 6000 : NEVER;
       if (K == 4) return 1200;
       if (K == 5) return D && !single ? NEVER : 600;
@@ -156,21 +170,25 @@ struct GenForms {
     constexpr int N = NEVER;
     // [FP64 two outputs, FP64 single, FP32 two outputs, FP32 single][degree]
     constexpr int to_2d[4][13] = {
-        {0, 65536, 0, 0, 6000, 0, 5500, 4096, 3000, 3000, 12000, 9000, 9000},
-        {0, N, 0, 32000, 6000, 11000, 5500, 7000, 3000, 3000, N, 16384, N},
-        {0, 0, 0, 0, 11000, 7500, 4096, 3584, 8192, 16384, 32768, 12000, N},
-        {0, 0, 0, 17000, 11000, 7500, 4096, 3584, 24000, N, N, N, N}};
-    constexpr int to_3d[4][10] = {{0, 0, 0, 0, 0, 2500, 576, 448, 1800, N},
-                                  {0, 0, 0, 0, 0, N, 576, 448, 2800, N},
-                                  {0, 0, 0, 0, 0, 800, 576, 3500, 1152, 448},
-                                  {0, 0, 0, 0, 0, 2000, 576, 6000, 1152, 448}};
+        {0, 65536, 0, 0, 5121, 0, 5500, 3500, 2600, 2500, 12000, 9000, 9000},
+        {0, N, 0, 16385, 5121, 5121, 5500, 3700, 2500, 2500, N, 12000, N},
+        {0, 0, 0, 0, 11000, 5121, 4096, 3584, 9100, 14500, 32768, 9800, N},
+        {0, 0, 0, 16385, 11000, 5121, 4096, 3584, 13000, N, N, N, N}};
+    constexpr int to_3d[4][10] = {{0, 0, 0, 0, 0, 2500, 576, 257, 1600, N},
+                                  {0, 0, 0, 0, 0, N, 576, 257, 2800, N},
+                                  {0, 0, 0, 0, 0, 800, 576, 3500, 950, 380},
+                                  {0, 0, 0, 0, 0, 2000, 576, 4800, 1152, 280}};
     const int row = (D ? 0 : 2) + (single ? 1 : 0);
     if constexpr (DIM == 2) return to_2d[row][K];
     else return to_3d[row][K];
   }
+  // launches whose line groups just fill the CUs once (four a CU) stay in the line form
+  static constexpr int ROUND =
+      DIM == 2 && (K == 8 || K == 9) && !D ? 1024 * GenShape<DIM, K>::CPB : 0;
   // (the node form's offsets into the vectors have 32 bits)
   static bool node(int n, bool single) {
     return n >= from(single) && n < to(single) &&
+           (single || n <= ROUND / 8 * 7 || n > ROUND) &&
            uint64_t(n) * (GenShape<DIM, K>::NF * GenShape<DIM, K>::ND) < (uint64_t(1) << 32);
   }
   static constexpr bool NODE_EXISTS = from(false) < to(false) || from(true) < to(true);

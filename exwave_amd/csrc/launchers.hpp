@@ -191,7 +191,7 @@ hipError_t launch_op(const DevMesh &m, const double *src, const double *tab,
     if (e.cell_list) return hipErrorInvalidValue;  // cell lists: Cartesian kernel only
     const int n = m.n_cells;
     if (n == 0) return hipSuccess;
-    const bool on = gen_kernel_enabled(), node = F::NODE_EXISTS && F::node(n, !e.o2);
+    const bool on = gen_kernel_enabled(), node = F::NODE_EXISTS && F::node(n, !e.o2 && !e.b);
     if constexpr (F::NODE_EXISTS && GenNodeShape<DIM, K>::ENABLED)
       if (on && node) {
         hipLaunchKernelGGL((dg_operator_gen_node_kernel<DIM, K, Number>), dim3(n),

@@ -1,6 +1,6 @@
 """The operator on general cells on both sides of every line between the form with
-one lane per node and the line form (they depend on degree, precision and the number
-of outputs; dg_operator_gen.hpp lists them): single sweeps and two-output sweeps
+one lane per node and the line form (they depend on degree, precision and whether
+the launch is a plain sweep; dg_operator_gen.hpp lists them): single sweeps and two-output sweeps
 with cell scales and a c operand, on vectors that are only 8-byte aligned, against
 the oracle.  Meshes whose last group is part-filled wherever a group has several cells."""
 import numpy as np
@@ -22,7 +22,14 @@ CASES = [(2, 1, 0, 173), (2, 1, 0, 174), (2, 1, 0, 224), (2, 1, 0, 257), (2, 3, 
          (2, 6, 1, 63), (2, 6, 1, 65), (2, 7, 1, 59), (2, 7, 1, 61), (2, 8, 1, 90),
          (2, 8, 1, 92), (2, 9, 1, 127), (2, 9, 1, 129), (2, 11, 1, 109), (2, 11, 1, 111),
          (2, 12, 1, 30), (3, 5, 1, 9), (3, 5, 1, 10), (3, 5, 1, 13), (3, 6, 1, 8), (3, 6, 1, 9),
-         (3, 7, 1, 15), (3, 7, 1, 16), (3, 8, 1, 10), (3, 8, 1, 11), (3, 9, 1, 7), (3, 9, 1, 8)]
+         (3, 7, 1, 15), (3, 7, 1, 16), (3, 8, 1, 10), (3, 8, 1, 11), (3, 9, 1, 7), (3, 9, 1, 8),
+         (2, 1, 0, 154), (2, 1, 0, 155), (2, 3, 0, 128), (2, 3, 0, 129), (2, 4, 0, 71),
+         (2, 4, 0, 72), (2, 5, 0, 71), (2, 5, 0, 72), (2, 7, 0, 59), (2, 7, 0, 61), (2, 8, 0, 50),
+         (2, 8, 0, 51), (2, 9, 0, 49), (2, 9, 0, 51), (2, 11, 0, 110), (3, 7, 0, 6),
+         (3, 8, 0, 11), (2, 3, 1, 129), (2, 5, 1, 71), (2, 5, 1, 72), (2, 8, 1, 79), (2, 8, 1, 80),
+         (2, 8, 1, 84), (2, 8, 1, 85), (2, 8, 1, 95), (2, 8, 1, 96), (2, 8, 1, 114), (2, 8, 1, 115),
+         (2, 9, 1, 73), (2, 9, 1, 74), (2, 9, 1, 78), (2, 9, 1, 79), (2, 9, 1, 120), (2, 9, 1, 121),
+         (2, 11, 1, 98), (2, 11, 1, 99), (3, 8, 1, 9), (3, 9, 1, 6)]
 
 
 @pytest.mark.parametrize("dim,k,fp32,nint", CASES)
