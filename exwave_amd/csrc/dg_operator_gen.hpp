@@ -145,7 +145,8 @@ struct GenSmall {
 // From a sweep in steps of 12 % of the cells, line form's time over the node form's just
 // below and above the line: FP64 2D k=4 5112 cells 1.15, 5700 0.78 (one round
 // of the node form's groups ends between), k=7 3248 1.02, 4095 0.96, k=8 2304 1.07, 2915
-// 0.97, k=9 2304 1.05, 2915 0.95, 3D k=7 252 1.22, 288 0.96, k=8 1573 1.02, 1728 0.97; FP32 2D k=8 9024 1.01, 10100 0.93,
+// 0.97, k=9 2304 1.05, 2915 0.95, 3D k=7 252 1.22, 288 0.96, k=8 1573 1.02, 1728 0.97;
+// FP32 2D k=8 9024 1.01, 10100 0.93,
 // k=9 14160 1.02, 15875 0.92, k=11 9024 1.05, 10100 0.96, 3D k=8 810 1.04, 1000 0.96, k=9 252
 // 1.16, 441 0.95.  FP32 2D k=8 and 9 just below one full round of the line form's groups: 5700
 // 1.02, 6399 0.93, 7140 0.86, 8010 1.00; 5112 1.05, 5700 0.95, 6399 1.21.  Plain sweeps: FP64 2D
